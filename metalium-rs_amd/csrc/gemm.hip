@@ -1808,10 +1808,11 @@ static int splitk_slices(const Plan &p) {
 }
 
 // Slices are multiples of 64 long, so with m and n multiples of 64 and k of
-// 32 every slice tiles exactly and the unguarded loads run.
+// the k-tile (32 F32 values, 64 BF16) every slice tiles exactly and the
+// unguarded loads run.
 template <typename T, typename SA, typename SB>
 static hipError_t run_splitk_kernels(const Plan &p, hipStream_t st) {
-  if (tiles_exactly(p, 64, 64, 32, 4)) return launch_orient<T, SA, SB, float, 64, 64, 2, 2, false>(p, st);
+  if (tiles_exactly(p, 64, 64, 128 / sizeof(T), 4)) return launch_orient<T, SA, SB, float, 64, 64, 2, 2, false>(p, st);
   return launch_orient<T, SA, SB, float, 64, 64, 2, 2, true>(p, st);
 }
 
