@@ -232,6 +232,9 @@ struct GemmArgs {
   // several copies of it (A = [hi | lo] parts of an F32 operand against one
   // B: B's k wraps modulo kb; 0 for none).
   int64_t kb = 0;
+  // Direct BF16 kernel, EDGE 2 only: A's k steps back by ka from k = ka0 on
+  // (0 for none).
+  int64_t ka = 0, ka0 = 0;
   // Direct BF16 kernel only: B's rows are gate|up pairs (32 gate rows, then
   // the 32 up rows of the same outputs, ...), and C receives silu(gate) * up
   // for the N / 2 outputs -- SWIGLU_PARTS: as its BF16 parts ([M, N] BF16: a
@@ -720,6 +723,7 @@ struct DmaOperand {
     // stored.  limit = 0: no edge.
     int64_t first_row, limit;
     const char *clamp;
+    uint32_t vclamp;  // the per-lane offset of a block read from `clamp`
   };
   // A wave's DMA instructions per tile: its blocks wave, wave + NW, ...;
   // where NW does not divide the blocks, a wave with one fewer repeats its
@@ -752,7 +756,7 @@ struct DmaOperand {
       base_off = ((k0 + RPB * wave) * ld + r0) * 2;
     }
     ustep = static_cast<int64_t>(RPB) * NW * ld * 2;
-    return Src{voff, reinterpret_cast<const char *>(src) + base_off, ustep, 0, 0, nullptr};
+    return Src{voff, reinterpret_cast<const char *>(src) + base_off, ustep, 0, 0, nullptr, voff};
   }
   // src_of for a k-contiguous operand of `rows` rows (a multiple of RPB) whose
   // last tile runs past them.
@@ -767,6 +771,32 @@ struct DmaOperand {
     return sr;
   }
 
+  // src_of for a tile that may run past an operand of any `rows` >= RPB (where
+  // they are contiguous, stored in whole chunks of 8): every lane past the
+  // last row, or chunk, reads the last one instead.  Those rows only feed
+  // results that are not stored.
+  template <int NW>
+  __device__ __forceinline__ static Src src_any(const uint16_t *src, int64_t ld, int64_t r0, int64_t k0, int wave,
+                                                int lane, int64_t rows) {
+    Src sr = src_of<NW>(src, ld, r0, k0, wave, lane);
+    const int lr = (lane * 16) / RB, pch = ((lane * 16) % RB) >> 4;
+    if constexpr (KCONTIG) {
+      // The last block of rows, whole or (rows not a multiple of RPB) partial.
+      const int part = static_cast<int>(rows % RPB);
+      const int64_t last = part ? rows - part : rows - RPB;
+      const int lrc = part && lr >= part ? part - 1 : lr;
+      sr.first_row = r0 + RPB * wave;
+      sr.limit = part ? last : rows;
+      sr.clamp = reinterpret_cast<const char *>(src) + (last * ld + k0) * 2;
+      sr.vclamp = static_cast<uint32_t>((lrc * ld + (pch ^ swz(lr)) * 8) * 2);
+    } else {
+      const int c = pch ^ (4 * ((RPB * wave + lr) & 3));
+      const int64_t cmax = (rows - r0 + 7) / 8 - 1;
+      sr.voff = static_cast<uint32_t>((lr * ld + (c < cmax ? c : cmax) * 8) * 2);
+    }
+    return sr;
+  }
+
   // The DMA instruction of this wave's block i of the tile into `lds`.
   template <int NW>
   __device__ __forceinline__ static void issue(const Src &sr, int i, char *lds, int wave) {
@@ -777,7 +807,11 @@ struct DmaOperand {
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void *)(lds)));
     const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds0 + b * 1024);
     const char *p = sr.base + i * sr.ustep;
-    if (sr.limit && sr.first_row + static_cast<int64_t>(i) * RPB * NW >= sr.limit) p = sr.clamp;
+    uint32_t voff = sr.voff;
+    if (sr.limit && sr.first_row + static_cast<int64_t>(i) * RPB * NW >= sr.limit) {
+      p = sr.clamp;
+      voff = sr.vclamp;
+    }
     const char *gb = reinterpret_cast<const char *>(
         static_cast<uint64_t>(static_cast<uint32_t>(
             __builtin_amdgcn_readfirstlane(static_cast<int>(reinterpret_cast<uintptr_t>(p))))) |
@@ -787,16 +821,26 @@ struct DmaOperand {
 #pragma clang diagnostic ignored "-Winline-asm"
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
-                 : "s"(m0v), "v"(sr.voff), "s"(gb)
+                 : "s"(m0v), "v"(voff), "s"(gb)
                  : "memory", "m0");
 #pragma clang diagnostic pop
   }
 
+  // The source of a tile whose last rows are taken as EDGE says (see
+  // gemm_pipe_body): whole tiles, whole blocks past the edge, or any rows.
+  template <int NW, int EDGE>
+  __device__ __forceinline__ static Src src_for(const uint16_t *src, int64_t ld, int64_t r0, int64_t k0, int wave,
+                                                int lane, int64_t rows) {
+    if constexpr (EDGE == 2) return src_any<NW>(src, ld, r0, k0, wave, lane, rows);
+    else if constexpr (EDGE == 1) return src_edge<NW>(src, ld, r0, k0, wave, lane, rows);
+    else return src_of<NW>(src, ld, r0, k0, wave, lane);
+  }
+
   // Issue this wave's share of the tile's 1 KiB blocks (all of them).
-  template <int NW>
+  template <int NW, int EDGE>
   __device__ __forceinline__ static void load(const uint16_t *src, int64_t ld, int64_t r0, int64_t k0, char *lds,
-                                              int wave, int lane, int64_t rows = 0) {
-    const Src sr = rows ? src_edge<NW>(src, ld, r0, k0, wave, lane, rows) : src_of<NW>(src, ld, r0, k0, wave, lane);
+                                              int wave, int lane, int64_t rows) {
+    const Src sr = src_for<NW, EDGE>(src, ld, r0, k0, wave, lane, rows);
 #pragma unroll
     for (int i = 0; i < per_wave<NW>(); ++i) issue<NW>(sr, i, lds, wave);
   }
@@ -1034,8 +1078,12 @@ __device__ __forceinline__ void qkv_tail(const GemmArgs &g, const f32x16 (&acc)[
   }
 }
 
-template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, bool GN>
+// EDGE 0: whole tiles.  1: the last column tile may run past N (B
+// k-contiguous, N a multiple of its block rows).  2: any M and N (rows of an
+// m/n-contiguous operand in multiples of 8); each result is stored by itself.
+template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, int EDGE>
 __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
+  constexpr int EDGE_A = EDGE == 2 ? 2 : 0;  // A's rows are whole tiles but for EDGE 2
   constexpr int BK = 32;  // two MFMA k steps per tile
   constexpr int NW = WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -1076,16 +1124,23 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
   // every thread issues PER_TILE DMA instructions per tile and the counted
   // waits stay exact.
   auto kclamp = [&](int64_t t) { return (t < ktiles ? t : ktiles - 1) * BK; };
-  // B's k of tile t: wrapped modulo its own extent when A repeats it.
-  auto kbof = [&](int64_t t) { return g.kb ? kclamp(t) % g.kb : kclamp(t); };
-  // GN: the last column tile runs past N (B k-contiguous, N a multiple of
-  // its block rows): those B rows are read from the last whole block, their
-  // results not stored.
-  const int64_t brows = GN ? g.N : 0;
+  // The operands' own k of tile t, where one repeats against the other's
+  // parts.  Only EDGE 2 steps A back too: the test in the whole tiles' loop
+  // cost 3% at 4096^3 (111.6 -> 115.2 us).
+  auto kaof = [&](int64_t t) {
+    const int64_t k = kclamp(t);
+    if constexpr (EDGE == 2) return g.ka && k >= g.ka0 ? k - g.ka : k;
+    else return k;
+  };
+  auto kbof = [&](int64_t t) {
+    const int64_t k = kclamp(t);
+    if constexpr (EDGE == 2) return g.kb && k >= g.kb ? k - g.kb : k;  // K <= 2 kb
+    else return g.kb ? k % g.kb : k;
+  };
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) {
-    OA::template load<NW>(A, g.lda, m0, kclamp(s), stages[s], wave, lane);
-    OB::template load<NW>(B, g.ldb, n0, kbof(s), stages[s] + OA::BYTES, wave, lane, brows);
+    OA::template load<NW, EDGE_A>(A, g.lda, m0, kaof(s), stages[s], wave, lane, g.M);
+    OB::template load<NW, EDGE>(B, g.ldb, n0, kbof(s), stages[s] + OA::BYTES, wave, lane, g.N);
   }
   // Tile 0 landed everywhere (tiles 1 .. NS-2 may be in flight).
   wait_vmcnt<(NS - 2) * PER_TILE>();
@@ -1118,9 +1173,8 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
         // their use (0.75 -> 0.85 of the MFMA cycles in the main loop at
         // 4096^3); whatever the step has no MFMA left for follows it.
         char *refill = stages[(s + NS - 1) % NS];
-        const auto sa = OA::template src_of<NW>(A, g.lda, m0, kclamp(kt + s + NS - 1), wave, lane);
-        const auto sb = GN ? OB::template src_edge<NW>(B, g.ldb, n0, kbof(kt + s + NS - 1), wave, lane, brows)
-                           : OB::template src_of<NW>(B, g.ldb, n0, kbof(kt + s + NS - 1), wave, lane);
+        const auto sa = OA::template src_for<NW, EDGE_A>(A, g.lda, m0, kaof(kt + s + NS - 1), wave, lane, g.M);
+        const auto sb = OB::template src_for<NW, EDGE>(B, g.ldb, n0, kbof(kt + s + NS - 1), wave, lane, g.N);
         const char *nst = stages[(s + 1) % NS];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1150,7 +1204,7 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
   // next to the accumulators.
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int64_t row0 = m0 + wm * WTM + 4 * lhalf, col0 = n0 + wn * WTN + lrow;
-  if constexpr (TN == 2) {
+  if constexpr (TN == 2 && EDGE < 2) {
     if (g.qkv.mode) {
       __syncthreads();  // every wave past its last read of the stages
       if (n0 < static_cast<int64_t>(g.qkv.heads + g.qkv.kvh) * 64) {  // a tile with RoPE heads
@@ -1161,7 +1215,7 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
       return;
     }
   }
-  if constexpr (TN % 2 == 0 && !GN) {
+  if constexpr (TN % 2 == 0 && EDGE == 0) {
     if (g.swiglu) {
       // Fragments (i, 2 jp) and (i, 2 jp + 1) are the gate and up columns of
       // outputs (n0 + wn WTN) / 2 + 32 jp + lane % 32: silu(gate) * up as the
@@ -1200,15 +1254,16 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      if (GN && col0 + j * 32 >= g.N) continue;
+      if (EDGE && col0 + j * 32 >= g.N) continue;
       TO *cij = C + (row0 + i * 32) * g.ldc + col0 + j * 32;
       float v[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) v[r] = acc[i][j][r];
-      if (!plain) fragment_epilogue<false>(g, row0 + i * 32, col0 + j * 32, v);
+      if (!plain) fragment_epilogue<EDGE == 2>(g, row0 + i * 32, col0 + j * 32, v);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int dr = 8 * (r >> 2) + (r & 3);
+        if (EDGE == 2 && row0 + i * 32 + dr >= g.M) continue;
         if constexpr (sizeof(TO) == 2) cij[dr * g.ldc] = f32_to_bf16_bits(v[r]);
         else cij[dr * g.ldc] = v[r];
       }
@@ -1217,17 +1272,17 @@ __device__ __forceinline__ void gemm_pipe_body(const GemmArgs &g) {
 }
 
 // Two waves per SIMD (8 per workgroup): at most 256 registers a wave.
-template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, bool GN>
+template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, int EDGE>
 __global__ void __launch_bounds__(WM *WN * 64) gemm_pipe_kernel(GemmArgs g) {
-  gemm_pipe_body<TO, BM, BN, NS, AK, BKC, WM, WN, GN>(g);
+  gemm_pipe_body<TO, BM, BN, NS, AK, BKC, WM, WN, EDGE>(g);
 }
 
 // One wave per SIMD (4 per workgroup): the whole 512-entry register file, so
 // a 128 x 128 wave tile keeps its accumulators in the AGPRs.
-template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, bool GN>
+template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, int EDGE>
 __global__ void __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_pipe1_kernel(GemmArgs g) {
-  gemm_pipe_body<TO, BM, BN, NS, AK, BKC, WM, WN, GN>(g);
+  gemm_pipe_body<TO, BM, BN, NS, AK, BKC, WM, WN, EDGE>(g);
 }
 
 // ------------------------------------------------- small-M products
@@ -1441,7 +1496,7 @@ struct Plan {
   int64_t ldc = 0;                // result row pitch (0: N)
   int64_t per_group = 0;          // items per group (0: one group of `batch`)
   int64_t sa2 = 0, sb2 = 0, sc2 = 0;  // group strides
-  int64_t kb = 0;  // direct BF16 kernel: B's k extent when A's k repeats it (see GemmArgs)
+  int64_t kb = 0, ka = 0, ka0 = 0;  // direct BF16 kernel: operands whose k repeats (see GemmArgs)
   int swiglu = 0;  // direct BF16 kernel: gate|up pairs into silu(gate) * up (see GemmArgs)
   QkvTail qkv;     // direct BF16 kernel: the q|k|v tail (see QkvTail)
   // The RMSNorm of the F32 result's rows (mi_linear_add_rms_norm): taken by
@@ -1485,7 +1540,7 @@ static hipError_t launch_cfg(const Plan &p, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, bool GN>
+template <typename TO, int BM, int BN, int NS, bool AK, bool BKC, int WM, int WN, int EDGE>
 static hipError_t launch_pipe_cfg(const Plan &p, hipStream_t st) {
   GemmArgs g;
   g.a = p.a; g.b = p.b; g.c = p.c;
@@ -1499,30 +1554,31 @@ static hipError_t launch_pipe_cfg(const Plan &p, hipStream_t st) {
   g.kc = 0;
   g.bias = p.bias; g.resid = p.resid; g.ldr = p.ldr;
   g.kb = p.kb;
+  g.ka = p.ka; g.ka0 = p.ka0;
   g.swiglu = p.swiglu;
   g.qkv = p.qkv;
-  g.tiles_m = static_cast<int>(p.M / BM);
+  g.tiles_m = static_cast<int>((p.M + BM - 1) / BM);
   g.tiles_n = static_cast<int>((p.N + BN - 1) / BN);
   dim3 grid(static_cast<unsigned>(g.tiles_m * g.tiles_n), static_cast<unsigned>(p.batch));
-  if constexpr (WM * WN == 4) gemm_pipe1_kernel<TO, BM, BN, NS, AK, BKC, WM, WN, GN><<<grid, 256, 0, st>>>(g);
-  else gemm_pipe_kernel<TO, BM, BN, NS, AK, BKC, WM, WN, GN><<<grid, WM * WN * 64, 0, st>>>(g);
+  if constexpr (WM * WN == 4) gemm_pipe1_kernel<TO, BM, BN, NS, AK, BKC, WM, WN, EDGE><<<grid, 256, 0, st>>>(g);
+  else gemm_pipe_kernel<TO, BM, BN, NS, AK, BKC, WM, WN, EDGE><<<grid, WM * WN * 64, 0, st>>>(g);
   return hipGetLastError();
 }
 
 template <typename TO, int BM, int BN, int NS, int WM, int WN>
 static hipError_t launch_pipe(const Plan &p, hipStream_t st) {
   const bool ak = !p.ta, bk = p.tb;
-  if (ak && bk) return launch_pipe_cfg<TO, BM, BN, NS, true, true, WM, WN, false>(p, st);
-  if (ak && !bk) return launch_pipe_cfg<TO, BM, BN, NS, true, false, WM, WN, false>(p, st);
-  if (!ak && bk) return launch_pipe_cfg<TO, BM, BN, NS, false, true, WM, WN, false>(p, st);
-  return launch_pipe_cfg<TO, BM, BN, NS, false, false, WM, WN, false>(p, st);
+  if (ak && bk) return launch_pipe_cfg<TO, BM, BN, NS, true, true, WM, WN, 0>(p, st);
+  if (ak && !bk) return launch_pipe_cfg<TO, BM, BN, NS, true, false, WM, WN, 0>(p, st);
+  if (!ak && bk) return launch_pipe_cfg<TO, BM, BN, NS, false, true, WM, WN, 0>(p, st);
+  return launch_pipe_cfg<TO, BM, BN, NS, false, false, WM, WN, 0>(p, st);
 }
 
 // A width that is not a multiple of the tile: B k-contiguous ([N, K] as the
 // weights are stored), N a multiple of 16, A k-contiguous.
 template <typename TO, int BM, int BN, int NS, int WM, int WN>
 static hipError_t launch_pipe_edge(const Plan &p, hipStream_t st) {
-  return launch_pipe_cfg<TO, BM, BN, NS, true, true, WM, WN, true>(p, st);
+  return launch_pipe_cfg<TO, BM, BN, NS, true, true, WM, WN, 1>(p, st);
 }
 
 
@@ -1665,7 +1721,7 @@ static hipError_t run_bf16(const Plan &p, hipStream_t st) {
       p.ldb % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15) &&
       tiles(128, 128) >= 128) {
     if (!parts_small_tiles(p)) {
-      if (pipe_192_fits(p)) return launch_pipe_cfg<TO, 256, 192, 5, true, true, 4, 2, false>(p, st);
+      if (pipe_192_fits(p)) return launch_pipe_cfg<TO, 256, 192, 5, true, true, 4, 2, 0>(p, st);
       return launch_pipe_edge<TO, 256, 256, 5, 2, 4>(p, st);
     }
     return launch_pipe_edge<TO, 128, 128, 5, 2, 2>(p, st);
@@ -1976,8 +2032,8 @@ static hipError_t launch_direct(const Plan &q, hipStream_t st) {
   if (q.N % 256 == 0)
     return bf ? launch_pipe<uint16_t, 256, 256, 5, 2, 4>(q, st) : launch_pipe<float, 256, 256, 5, 2, 4>(q, st);
   if (pipe_192_fits(q))
-    return bf ? launch_pipe_cfg<uint16_t, 256, 192, 5, true, true, 4, 2, false>(q, st)
-              : launch_pipe_cfg<float, 256, 192, 5, true, true, 4, 2, false>(q, st);
+    return bf ? launch_pipe_cfg<uint16_t, 256, 192, 5, true, true, 4, 2, 0>(q, st)
+              : launch_pipe_cfg<float, 256, 192, 5, true, true, 4, 2, 0>(q, st);
   return bf ? launch_pipe_edge<uint16_t, 256, 256, 5, 2, 4>(q, st) : launch_pipe_edge<float, 256, 256, 5, 2, 4>(q, st);
 }
 
@@ -2007,9 +2063,263 @@ static int run_stacked_split(mi_ctx *ctx, const Plan &p) {
   return check_launch(ctx, "matmul");
 }
 
+// ------------------------------------- any shape on the direct BF16 kernel
+// The direct kernel reads BF16 operands by 16-byte DMA in whole k-tiles of
+// 32.  Operands that do not lie so -- F32 ones, taken as their BF16 parts in
+// the fast mode; a k that 32 does not divide; rows off 16-byte boundaries; a
+// transposed A -- are first written once in that form (k zero-padded), and
+// the rows and columns past M and N are the kernel's edge (EDGE 2).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
+
+// Eight elements from p (any element alignment), zeros past `valid`, as their
+// BF16 heads and, for F32, remainders.
+template <typename S>
+__device__ __forceinline__ void pack8(const S *p, int valid, uint4 &hi, uint4 &lo) {
+  if constexpr (sizeof(S) == 4) {
+    float v[8];
+    if (valid >= 8) {
+      const f32x4u a = *reinterpret_cast<const f32x4u *>(p), b = *reinterpret_cast<const f32x4u *>(p + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = e < valid ? p[e] : 0.0f;
+    }
+    split_bf16x2(v[0], v[1], hi.x, lo.x);
+    split_bf16x2(v[2], v[3], hi.y, lo.y);
+    split_bf16x2(v[4], v[5], hi.z, lo.z);
+    split_bf16x2(v[6], v[7], hi.w, lo.w);
+  } else {
+    u16x8u v;
+    if (valid >= 8) {
+      v = *reinterpret_cast<const u16x8u *>(p);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = e < valid ? p[e] : uint16_t(0);
+    }
+    hi = __builtin_bit_cast(uint4, v);
+  }
+}
+
+struct PackArgs {
+  const void *src;
+  uint16_t *dst;
+  int64_t rows, cols, ld, item;     // the source: valid rows and columns, pitch, item stride
+  int64_t drows, dcols, dld, ditem; // the result: padded extent, pitch, item stride
+  int64_t hi, lo;                   // offsets of the heads' and the remainders' copies
+};
+
+// A row-major operand into its padded BF16 form, eight elements a thread:
+// bound by HBM (4 bytes read and 4 written an F32 element).
+template <typename S>
+__global__ void __launch_bounds__(256) pack_rows_kernel(PackArgs g) {
+  const int64_t per_row = g.dcols / 8, n = g.drows * per_row;
+  const int64_t u = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (u >= n) return;
+  const int64_t r = u / per_row, c = (u - r * per_row) * 8;
+  const S *src = static_cast<const S *>(g.src) + blockIdx.y * g.item + r * g.ld + c;
+  const int64_t left = r < g.rows ? g.cols - c : 0;
+  uint4 hi, lo;
+  pack8<S>(src, left < 0 ? 0 : (left > 8 ? 8 : static_cast<int>(left)), hi, lo);
+  uint16_t *dst = g.dst + blockIdx.y * g.ditem + r * g.dld + c;
+  *reinterpret_cast<uint4 *>(dst + g.hi) = hi;
+  if constexpr (sizeof(S) == 4) *reinterpret_cast<uint4 *>(dst + g.lo) = lo;
+}
+
+// The same for a transposed operand: source [cols of the result][rows], 64 x
+// 64 elements a block through LDS (a pitch of 65 words keeps both the rows'
+// writes and the columns' reads off each other's banks).
+template <typename S>
+__global__ void __launch_bounds__(256) pack_transposed_kernel(PackArgs g) {
+  __shared__ float tile[64][65];
+  const int t = threadIdx.x;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * 64, r0 = static_cast<int64_t>(blockIdx.y) * 64;
+  const S *src = static_cast<const S *>(g.src) + blockIdx.z * g.item;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {  // source row c0 + 4 i + t / 64, its elements r0 + t % 64
+    const int64_t c = c0 + 4 * i + (t >> 6), r = r0 + (t & 63);
+    float v = 0.0f;
+    if (c < g.cols && r < g.rows) {
+      if constexpr (sizeof(S) == 4) v = src[c * g.ld + r];
+      else v = bf16_bits_to_f32(src[c * g.ld + r]);
+    }
+    tile[4 * i + (t >> 6)][t & 63] = v;
+  }
+  __syncthreads();
+  const int64_t r = r0 + (t >> 2);
+  if (r >= g.drows) return;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t c = c0 + 16 * (t & 3) + 8 * h;
+    if (c >= g.dcols) continue;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = tile[16 * (t & 3) + 8 * h + e][t >> 2];
+    uint4 hi, lo;
+    pack8<float>(v, 8, hi, lo);  // BF16 values: their heads are themselves
+    uint16_t *dst = g.dst + blockIdx.z * g.ditem + r * g.dld + c;
+    *reinterpret_cast<uint4 *>(dst + g.hi) = hi;
+    if constexpr (sizeof(S) == 4) *reinterpret_cast<uint4 *>(dst + g.lo) = lo;
+  }
+}
+
+// One operand's packed form: `rows` x `k` elements of kind `elem`, k
+// contiguous in the result (else its rows are, k by k), from a source that
+// has its k contiguous or not.  Parts side by side along k: the heads first,
+// or last where `lo_first`.
+static hipError_t pack_operand(hipStream_t st, const void *src, int elem, bool src_kcontig, bool dst_kcontig,
+                               int64_t rows, int64_t k, int64_t kp, int64_t ld, int64_t item, int64_t items,
+                               bool lo_first, uint16_t *dst, int64_t *dst_ld, int64_t *dst_item) {
+  const int parts = elem == MI_F32 ? 2 : 1;
+  PackArgs g;
+  g.src = src; g.dst = dst;
+  g.ld = ld; g.item = item;
+  int64_t part;  // elements between the two copies
+  if (dst_kcontig) {
+    g.rows = g.drows = rows; g.cols = k; g.dcols = kp;
+    g.dld = parts * kp; g.ditem = rows * g.dld;
+    part = kp;
+  } else {
+    g.rows = k; g.drows = kp; g.cols = rows; g.dcols = (rows + 7) / 8 * 8;
+    g.dld = g.dcols; g.ditem = parts * kp * g.dld;
+    part = kp * g.dld;
+  }
+  g.hi = lo_first && parts == 2 ? part : 0;
+  g.lo = lo_first ? 0 : part;
+  *dst_ld = g.dld;
+  *dst_item = g.ditem;
+  if (src_kcontig == dst_kcontig) {
+    const dim3 grid(static_cast<unsigned>((g.drows * (g.dcols / 8) + 255) / 256), static_cast<unsigned>(items));
+    if (elem == MI_F32) pack_rows_kernel<float><<<grid, 256, 0, st>>>(g);
+    else pack_rows_kernel<uint16_t><<<grid, 256, 0, st>>>(g);
+  } else {
+    const dim3 grid(static_cast<unsigned>((g.dcols + 63) / 64), static_cast<unsigned>((g.drows + 63) / 64),
+                    static_cast<unsigned>(items));
+    if (elem == MI_F32) pack_transposed_kernel<float><<<grid, 256, 0, st>>>(g);
+    else pack_transposed_kernel<uint16_t><<<grid, 256, 0, st>>>(g);
+  }
+  return hipGetLastError();
+}
+
+template <typename TO, bool BKC>
+static hipError_t launch_any_tile(const Plan &q, hipStream_t st) {
+  const bool whole = !q.ka;  // the whole-tile form reads A's k as it lies
+  const int64_t t256 = ((q.M + 255) / 256) * ((q.N + 255) / 256) * q.batch;
+  if (t256 >= 192) {
+    if (whole && q.M % 256 == 0 && q.N % 256 == 0) return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 0>(q, st);
+    return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 2>(q, st);
+  }
+  if (whole && q.M % 128 == 0 && q.N % 128 == 0) return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 0>(q, st);
+  return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 2>(q, st);
+}
+
+// The BF16 products that run_bf16 sends to the direct kernel as they lie.
+static bool exactly_direct(const Plan &p) {
+  if (p.ea != MI_BF16 || p.eb != MI_BF16) return false;
+  if (tiles_exactly(p, 128, 128, 32, 8)) return true;
+  return p.batch == 1 && !p.ta && p.tb && p.N % 16 == 0 && p.M % 128 == 0 && p.K % 32 == 0 && p.lda % 8 == 0 &&
+         p.ldb % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15) &&
+         ((p.M + 127) / 128) * ((p.N + 127) / 128) >= 128;
+}
+
+// Whether a product goes to the direct kernel through packed operands.  Both
+// sides of each line measured (us, this path after what ran before):
+//  * F32 x F32 in the fast mode, where it splits (2^33 multiply-adds, 128
+//    tiles; below that F32 products keep the F32 matrix cores' precision):
+//    4096^3 992 -> 372 (370 TF/s), 4095^3 1790 -> 384, 3001 x 2500 x 2047
+//    431 -> 140.  The split kernel converts every tile again for each block
+//    that reads it, with no k-tile in flight behind the one it multiplies.
+//  * F32 activations x BF16: 4000 x 4000 x 3000 674 -> 193, 1500 x 3072 x 768
+//    93 -> 42; 2000 x 576 x 1536 37.7 -> 40.0, below the line at 2^31.
+//  * BF16 off the whole tiles: 2001^3 450 -> 38.8, 4095 x 4097 x 4001 1719 ->
+//    215 (transposed A 5180 -> 217), 1000^3 42.6 -> 21.3, 700^3 29.2 -> 17.1;
+//    100 x 3000 x 1000 (24 tiles) 16.4 -> 20.9 and 512 x 512 x 500 (16 tiles)
+//    19.8 -> 12.7 lie below the line at 32 tiles.
+static bool direct_any_pays(const Plan &p) {
+  if (p.per_group || p.kc || p.swiglu || p.qkv.mode || p.M < 16 || p.N < 16) return false;
+  const bool f32 = p.ea == MI_F32 || p.eb == MI_F32;
+  if (f32 && !p.fast) return false;
+  if (p.K >= (int64_t(1) << 24) || p.lda >= (int64_t(1) << 26) || p.ldb >= (int64_t(1) << 26)) return false;
+  const int64_t macs = p.M * p.N * p.K * p.batch;
+  const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+  if (!f32) return macs >= (int64_t(1) << 28) && t128 >= 32;
+  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return macs >= (int64_t(1) << 31) && t128 >= 128;
+  return macs >= (int64_t(1) << 33) && t128 >= 128;
+}
+
+// The product through packed operands; *ran stays false (and nothing is
+// launched) where their scratch cannot be had.
+static int run_direct_any(mi_ctx *ctx, const Plan &p, bool *ran) {
+  *ran = false;
+  Plan q = p;
+  const int na = p.ea == MI_F32 ? 2 : 1, nb = p.eb == MI_F32 ? 2 : 1;
+  const int64_t kp = (p.K + 31) / 32 * 32;
+  auto lies = [&](const void *x, int64_t ld, int64_t item) {
+    return p.K % 32 == 0 && ld % 8 == 0 && item % 8 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15);
+  };
+  const bool a_in = na == 1 && !p.ta && lies(p.a, p.lda, p.sa);
+  const bool b_in = nb == 1 && (p.tb || p.N % 8 == 0) && lies(p.b, p.ldb, p.sb);
+  const int64_t ia = p.sa ? p.batch : 1, ib = p.sb ? p.batch : 1;
+  const int64_t n8 = (p.N + 7) / 8 * 8;
+  mi_id aid = 0, bid = 0;
+  Buffer *ab = nullptr, *bb = nullptr;
+  if (!a_in && new_buffer(ctx, ia * p.M, na * kp, MI_BF16, &aid, &ab)) return MI_OK;
+  if (!b_in && new_buffer(ctx, ib * nb * kp, p.tb ? p.N : n8, MI_BF16, &bid, &bb)) {
+    if (aid) mi_free(ctx, aid);
+    return MI_OK;
+  }
+  if (aid) ab = lookup(ctx, aid);
+  hipError_t e = hipSuccess;
+  if (!a_in) {
+    e = pack_operand(ctx->stream, p.a, p.ea, !p.ta, true, p.M, p.K, kp, p.lda, p.sa, ia, nb == 2,
+                     static_cast<uint16_t *>(ab->ptr), &q.lda, &q.sa);
+    q.a = ab->ptr;
+    if (ia == 1) q.sa = 0;
+  }
+  if (!b_in && e == hipSuccess) {
+    e = pack_operand(ctx->stream, p.b, p.eb, p.tb, p.tb, p.N, p.K, kp, p.ldb, p.sb, ib, false,
+                     static_cast<uint16_t *>(bb->ptr), &q.ldb, &q.sb);
+    q.b = bb->ptr;
+    if (ib == 1) q.sb = 0;
+  }
+  q.ea = q.eb = MI_BF16;
+  q.ta = false;
+  q.K = kp;
+  if (na == 2 && nb == 2) {
+    // lo_a hi_b, hi_a lo_b, then hi_a hi_b, the small sums first.
+    q.K = 3 * kp;
+    q.ka = kp; q.ka0 = 2 * kp;
+    q.kb = 2 * kp;
+  } else if (na == 2) {  // hi_a b, then lo_a b
+    q.K = 2 * kp;
+    q.kb = kp;
+  } else if (nb == 2) {
+    q.K = 2 * kp;
+    q.ka = q.ka0 = kp;
+  }
+  if (e == hipSuccess) {
+    if (p.eo == MI_BF16)
+      e = p.tb ? launch_any_tile<uint16_t, true>(q, ctx->stream) : launch_any_tile<uint16_t, false>(q, ctx->stream);
+    else
+      e = p.tb ? launch_any_tile<float, true>(q, ctx->stream) : launch_any_tile<float, false>(q, ctx->stream);
+  }
+  // Stream-ordered: the blocks are reused only by later work.
+  if (aid) mi_free(ctx, aid);
+  if (bid) mi_free(ctx, bid);
+  *ran = true;
+  if (e != hipSuccess) return fail(ctx, MI_E_HIP, "matmul launch: %s", hipGetErrorString(e));
+  return check_launch(ctx, "matmul");
+}
+
 static int run_product(mi_ctx *ctx, Plan &p) {
   hipError_t e;
   if (stacked_split_pays(p)) return run_stacked_split(ctx, p);
+  if (direct_any_pays(p) && !exactly_direct(p)) {
+    bool ran;
+    const int s = run_direct_any(ctx, p, &ran);
+    if (s || ran) return s;
+  }
   if (gemv_fits(p)) {
     launch_gemv(p, ctx->stream);
     e = hipGetLastError();

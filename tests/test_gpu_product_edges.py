@@ -28,3 +28,75 @@ def test_bf16_split_k_of_a_half_k_tile(engine, m, n, k):
     for t in (ia, ib, o):
         engine.free(t)
     assert np.array_equal(got, (a.astype(np.float64) @ b).astype(np.float32))
+
+
+# Shapes that reach the direct kernel through packed operands: each edge of
+# its 256 x 256 and 128 x 128 tiles, k off the k-tile, both orientations,
+# in-place operands whose rows end mid-block or mid-tile, BF16 results.
+@pytest.mark.parametrize("m,n,k,ta,tb,out", [
+    (1000, 1000, 1000, False, False, "f32"),   # k % 32, packed both
+    (1001, 1023, 512, False, True, "f32"),     # in place, rows off the DMA's blocks
+    (1001, 1016, 512, False, False, "f32"),    # in place, columns in eights
+    (777, 2049, 257, False, False, "bf16"),    # odd pitch, one column past a tile
+    (513, 1025, 640, True, False, "f32"),      # transposed A
+    (3585, 3841, 96, True, True, "f32"),       # 256-row tiles, one past the last
+])
+def test_bf16_any_shape(engine, m, n, k, ta, tb, out):
+    a, b = _ints((k, m) if ta else (m, k)), _ints((n, k) if tb else (k, n))
+    ia, ib = engine.upload_bf16(bf16_bits(a)), engine.upload_bf16(bf16_bits(b))
+    o = engine.matmul_dram(ia, ta, ib, tb, miburn.BF16 if out == "bf16" else miburn.F32)
+    got = engine.download(o)
+    for t in (ia, ib, o):
+        engine.free(t)
+    want = ((a.T if ta else a) @ (b.T if tb else b)).astype(np.float32)  # exact: |sums| < 2^24
+    if out == "bf16":
+        got, want = got, bf16_bits(want)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("bcast", ["none", "a", "b"])
+def test_bf16_any_shape_batched(engine, bcast):
+    bt, m, n, k = 6, 500, 490, 250
+    a, b = _ints((1 if bcast == "a" else bt, m, k)), _ints((1 if bcast == "b" else bt, k, n))
+    ia = engine.upload_bf16(bf16_bits(a.reshape(-1, k)))
+    ib = engine.upload_bf16(bf16_bits(b.reshape(-1, n)))
+    o = engine.matmul_dram_batched(ia, False, ib, False, bt, m, k, n)
+    got = engine.download(o).reshape(bt, m, n)
+    for t in (ia, ib, o):
+        engine.free(t)
+    assert np.array_equal(got, np.matmul(a, b))
+
+
+@pytest.mark.parametrize("ea,eb,m,n,k,ta,tb", [
+    ("f32", "f32", 2051, 2049, 2050, False, False),
+    ("f32", "f32", 2051, 2049, 2050, True, True),
+    ("bf16", "f32", 2051, 2049, 2050, False, True),
+    ("f32", "bf16", 1501, 2051, 800, False, True),
+    ("f32", "bf16", 1501, 2050, 801, True, False),
+])
+def test_f32_any_shape_fast(engine, ea, eb, m, n, k, ta, tb):
+    """The fast mode's parts: error per product within 3 * 2^-18 |a||b| and the
+    F32 accumulation's 2 K * 2^-24, each against sum |a||b|."""
+    a, b = (RNG.standard_normal(s).astype(np.float32) for s in ((k, m) if ta else (m, k), (n, k) if tb else (k, n)))
+    up = {"f32": engine.upload, "bf16": lambda x: engine.upload_bf16(bf16_bits(x))}
+    av, bv = (x if e == "f32" else bf16_to_f32(bf16_bits(x)) for x, e in ((a, ea), (b, eb)))
+    ia, ib = up[ea](a), up[eb](b)
+    o = engine.matmul_dram(ia, ta, ib, tb)
+    got = engine.download(o)
+    for t in (ia, ib, o):
+        engine.free(t)
+    av, bv = (av.T if ta else av).astype(np.float64), (bv.T if tb else bv).astype(np.float64)
+    bound = (3 * 2.0 ** -18 + 2 * k * 2.0 ** -24) * (np.abs(av) @ np.abs(bv))
+    assert np.all(np.abs(got - av @ bv) <= bound)
+
+
+def test_f32_any_shape_bias_residual(engine):
+    m, n, k = 1501, 2051, 801
+    x, w = _ints((m, k)), _ints((n, k))
+    bias, res = _ints((1, n)), _ints((m, n))
+    ids = [engine.upload(x), engine.upload_bf16(bf16_bits(w)), engine.upload(bias), engine.upload(res)]
+    o = engine.linear(ids[0], ids[1], True, ids[2], ids[3])
+    got = engine.download(o)
+    for t in ids + [o]:
+        engine.free(t)
+    assert np.array_equal(got, res + (x @ w.T + bias))
