@@ -100,3 +100,61 @@ def test_f32_any_shape_bias_residual(engine):
     for t in ids + [o]:
         engine.free(t)
     assert np.array_equal(got, res + (x @ w.T + bias))
+
+
+# F32 products at F32 precision: each tile (64 x 64, 64 x 128, 128 x 128),
+# whole and with edges, each DMA width, k-tile remainders, one k-tile, slices.
+F32_SHAPES = [(64, 64, 32), (64, 64, 8), (65, 67, 33), (1, 1, 1), (130, 66, 20), (128, 192, 96), (512, 512, 512),
+              (2048, 768, 256), (2050, 772, 260), (2049, 771, 259), (2048, 2048, 64), (2052, 2044, 68),
+              (257, 129, 2047), (1500, 1500, 300)]
+
+
+def _f32_product(engine, a, ta, b, tb):
+    ia, ib = engine.upload(a), engine.upload(b)
+    o = engine.matmul_dram(ia, ta, ib, tb)
+    got = engine.download(o)
+    for t in (ia, ib, o):
+        engine.free(t)
+    return got
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,n,k", F32_SHAPES)
+def test_f32_precise_product(engine, m, n, k, ta, tb):
+    """Against float64 within an F32 sum's bound, k + 4 roundings of 2^-24 of
+    sum |a||b| (the parts left out of a product: 2^-24 of it)."""
+    a, b = (RNG.standard_normal(s).astype(np.float32) for s in ((k, m) if ta else (m, k), (n, k) if tb else (k, n)))
+    got = _f32_product(engine, a, ta, b, tb)
+    av, bv = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+    assert np.all(np.abs(got - av @ bv) <= (k + 4) * 2.0 ** -24 * (np.abs(av) @ np.abs(bv)))
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 64, 40), (1024, 2048, 256), (2048, 2048, 64)])
+def test_f32_non_finite_operands(engine, m, n, k):
+    """An infinity, a NaN, a value next to the largest and zeros against them
+    give what F32 arithmetic gives, also where parts are multiplied."""
+    a, b = RNG.standard_normal((m, k)).astype(np.float32), RNG.standard_normal((k, n)).astype(np.float32)
+    a[3, 5], a[7, 1], a[9, 2], a[m - 1, k - 1] = np.inf, np.nan, np.float32(3.4028e38), -np.inf
+    b[5, 4] = b[2, 11] = 0.0
+    b[2, :8] = 0.25
+    got = _f32_product(engine, a, False, b, False)
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        want = np.where(np.abs(want) > np.finfo(np.float32).max, np.copysign(np.inf, want), want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32)) and not np.isinf(got[~inf]).any()
+    row9 = np.isfinite(want[9])
+    assert np.allclose(got[9][row9], want[9][row9], rtol=1e-6)
+
+
+def test_f32_sum_has_no_bias(engine):
+    """A sum over the rows of a product of parts: its error is the rounding
+    errors' sum, not their number times a bias (2e-8 of a value each)."""
+    m, n, k = 2048, 2048, 512
+    a, b = RNG.standard_normal((m, k)).astype(np.float32), RNG.standard_normal((k, n)).astype(np.float32)
+    d = _f32_product(engine, a, False, b, False) - a.astype(np.float64) @ b.astype(np.float64)
+    sd = d.std()
+    assert abs(d.mean()) < 6 * sd / np.sqrt(m * n)                       # independent errors' mean
+    assert np.abs(d.mean(axis=0)).max() < 7 * sd / np.sqrt(m)            # and each column's
