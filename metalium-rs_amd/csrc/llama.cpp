@@ -15,7 +15,7 @@
 // step of at most 32 sequences runs six fused launches a layer -- RMSNorm +
 // q|k|v + RoPE + cache write, attention (two), o + residual, RMSNorm +
 // gate|up + SiLU-mul, down + residual.  The KV cache of a layer is
-// [batch * kv_heads * max_ctx, head_dim], item (sequence, kv head), F32 under
+// [batch * kv_heads * cap, head_dim], item (sequence, kv head), F32 under
 // the reference numeric contract and BF16 under the performance one (which
 // also rounds a prefill product's activation operand to BF16), so the
 // attention of a query group is one product over a block of the cache:
@@ -82,7 +82,7 @@ struct mi_llama {
   mi_llama_config cfg;
   Tensor embed, final_norm;
   std::vector<Layer> layers;
-  Tensor rope_cos, rope_sin;  // [max_ctx, head_dim]
+  Tensor rope_cos, rope_sin;  // [cap, head_dim]
   int64_t len = 0;            // positions in the cache
   int64_t cache_batch = 0;    // sequences the cache holds
   // Traced decode steps over the current caches, by span; their inputs: the
@@ -138,6 +138,15 @@ constexpr int64_t kSpanStep = 64;
 // 32 x 64) output tile with k split over its waves, the activations handed
 // over in tiles by the norms and the SwiGLU.
 constexpr int64_t kTilesMaxRows = 2048;
+// New positions from which a prompt is padded to run on them.
+constexpr int64_t kPadMinT = 17;
+// Rows from which the fast mode splits F32 activations against BF16 weights.
+constexpr int64_t kSplitMinRows = 256;
+
+// The caches and rotary tables hold max_ctx positions rounded up to this, so
+// that a prompt reaching max_ctx can be run a few padding positions longer.
+constexpr int64_t kCapStep = 32;
+int64_t cache_cap(const mi_llama_config &c) { return (c.max_ctx + kCapStep - 1) / kCapStep * kCapStep; }
 
 int64_t decode_span(const mi_llama *m, int64_t ctxlen) {
   return std::min<int64_t>(m->cfg.max_ctx, (ctxlen + kSpanStep - 1) / kSpanStep * kSpanStep);
@@ -189,17 +198,13 @@ static bool parts_pay(mi_ctx *ctx, int64_t rows, int64_t k, int64_t n) {
   return rows >= 4096 && rows % 128 == 0 && k % 32 == 0 && n % 16 == 0;
 }
 
-// The forward of `t` positions per sequence at cache length m->len; returns
-// the hidden states [batch * t, hidden] before the final norm.
-// The hidden rows of token ids already on the device ([batch * t] I32, rows
-// (sequence, position)).
 // A prefill's attention over q from the q|k|v tail (rows (sequence,
 // position, head) for the fused kernel, else regrouped per kv head): the
 // output rows (sequence, position) of heads x head_dim.
 Tensor attention_of(mi_llama *m, Layer &L, const Tensor &q, int64_t batch, int64_t t, int64_t pos0, int64_t ctxlen,
                     bool fused, const Tensor &mask, float scale) {
   const mi_llama_config &c = m->cfg;
-  const int64_t H = c.heads, KVH = c.kv_heads, D = c.head_dim, G = H / KVH, maxc = c.max_ctx, rows = batch * t;
+  const int64_t H = c.heads, KVH = c.kv_heads, D = c.head_dim, G = H / KVH, maxc = cache_cap(c), rows = batch * t;
   if (fused) return burn::attention_rows(q.reshape({rows, H * D}), L.cache_k, L.cache_v, batch, t, H, KVH, pos0, scale);
   // [batch * KVH * t * G, D], rows (p, g) of each (sequence, kv head)
   Tensor scores = burn::matmul_blocks(q, false, L.cache_k, true, batch * KVH, t * G, D, ctxlen, 0, t * G * D, 0,
@@ -213,7 +218,46 @@ Tensor attention_of(mi_llama *m, Layer &L, const Tensor &q, int64_t batch, int64
   return burn::copy4(o, dims, 0, st).reshape({rows, H * D});
 }
 
+// The positions a sequence runs of a prompt of t, at cache length pos0: t, or
+// the fewest more that make the rows a multiple of 32 where those run the
+// tiled weights (kTilesMaxRows).  The padding rows follow each sequence's own
+// positions, which never attend to them; their cache rows lie past the length
+// and are written again before they are read.  Under the reference contract
+// from 256 rows, where the products take the activations in two BF16 parts
+// either way (fewer rows off the tiles run at F32 precision, and stay there).
+// SmolLM2 prompts, ms: reference 500 tokens 3.35 -> 1.85, 4 x 150 3.49 -> 1.93;
+// performance 500 2.38 -> 1.61, 69 1.90 -> 1.24, 17 1.70 -> 1.11 (unpadded: the
+// guarded products, split over k, the RoPE tail and the SwiGLU by themselves).
+int64_t padded_positions(const mi_llama *m, int64_t batch, int64_t t, int64_t pos0) {
+  const mi_llama_config &c = m->cfg;
+  if (t < kPadMinT || m->layers.empty() || !m->layers[0].t_wqkv.defined()) return t;
+  int mode = MI_MATMUL_FAST;
+  (void)mi_get_matmul_mode(m->ctx, &mode);
+  if (c.numerics != MI_NUMERICS_PERFORMANCE && (mode != MI_MATMUL_FAST || batch * t < kSplitMinRows)) return t;
+  int64_t tp = t;
+  while (batch * tp % 32) ++tp;
+  return batch * tp <= kTilesMaxRows && pos0 + tp <= cache_cap(c) ? tp : t;
+}
+
+Tensor forward_rows(mi_llama *m, Tensor x, int64_t batch, int64_t t);
+
+// The hidden rows of token ids already on the device ([batch * t] I32, rows
+// (sequence, position)), before the final norm.
 Tensor forward_ids(mi_llama *m, const Tensor &idx, int64_t batch, int64_t t) {
+  const int64_t hid = m->cfg.hidden, pos0 = m->len, tp = padded_positions(m, batch, t, pos0);
+  Tensor x = burn::select_rows_as(m->embed, idx, MI_F32);  // [rows, hidden], the BF16 rows widened
+  x = x.reshape({batch * t, hid});
+  if (tp == t) return forward_rows(m, x, batch, t);
+  const int64_t dims[4] = {1, batch, t, hid}, real[4] = {0, t * hid, hid, 1}, pad[4] = {0, tp * hid, hid, 1};
+  Tensor xp = burn::fill(m->ctx, {batch * tp, hid}, MI_F32, 0);
+  burn::copy_into4(xp, 0, pad, x, 0, real, dims);
+  x = forward_rows(m, xp, batch, tp);
+  m->len = pos0 + t;
+  return burn::copy4(x, dims, 0, pad).reshape({batch * t, hid});
+}
+
+// The forward of the embedded rows x [batch * t, hidden] at the cache's length.
+Tensor forward_rows(mi_llama *m, Tensor x, int64_t batch, int64_t t) {
   mi_ctx *ctx = m->ctx;
   const mi_llama_config &c = m->cfg;
   const int64_t H = c.heads, KVH = c.kv_heads, D = c.head_dim, G = H / KVH;
@@ -222,8 +266,6 @@ Tensor forward_ids(mi_llama *m, const Tensor &idx, int64_t batch, int64_t t) {
 
   // The element type of a prefill product's activation operand.
   const int act = c.numerics == MI_NUMERICS_PERFORMANCE ? MI_BF16 : MI_F32;
-  Tensor x = burn::select_rows_as(m->embed, idx, MI_F32);  // [rows, hidden], the BF16 rows widened
-  x = x.reshape({rows, c.hidden});
 
   // A few new positions (decode) take the fused attention kernel, and so does
   // a long prompt with 64-wide heads (the matrix-core flash kernel behind
@@ -424,8 +466,8 @@ void ensure_cache(mi_llama *m, int64_t batch) {
       // The old caches go before the new ones are made, so their memory is reused.
       L.cache_k = Tensor();
       L.cache_v = Tensor();
-      L.cache_k = burn::fill(m->ctx, {batch * c.kv_heads * c.max_ctx, c.head_dim}, kv, 0);
-      L.cache_v = burn::fill(m->ctx, {batch * c.kv_heads * c.max_ctx, c.head_dim}, kv, 0);
+      L.cache_k = burn::fill(m->ctx, {batch * c.kv_heads * cache_cap(c), c.head_dim}, kv, 0);
+      L.cache_v = burn::fill(m->ctx, {batch * c.kv_heads * cache_cap(c), c.head_dim}, kv, 0);
     }
     m->cache_batch = batch;
   }
@@ -495,8 +537,9 @@ int mi_llama_create(mi_ctx *ctx, const mi_llama_config *cfg, uint64_t seed, floa
     // Rotary tables (rope.rs:14-60): angle = position * theta^(-2i / d), the
     // first half repeated as the second, sin's first half negated.
     const int64_t D = c.head_dim, half = D / 2;
-    std::vector<float> cs(static_cast<size_t>(c.max_ctx * D)), sn(cs.size());
-    for (int64_t p = 0; p < c.max_ctx; ++p)
+    const int64_t cap = cache_cap(c);
+    std::vector<float> cs(static_cast<size_t>(cap * D)), sn(cs.size());
+    for (int64_t p = 0; p < cap; ++p)
       for (int64_t i = 0; i < half; ++i) {
         const float freq = static_cast<float>(std::pow(static_cast<double>(c.rope_theta), -2.0 * i / D));
         const float ang = static_cast<float>(p) * freq;
@@ -507,8 +550,8 @@ int mi_llama_create(mi_ctx *ctx, const mi_llama_config *cfg, uint64_t seed, floa
         sn[p * D + i] = -si;
         sn[p * D + half + i] = si;
       }
-    m->rope_cos = burn::float_from_data(ctx, cs.data(), {c.max_ctx, D});
-    m->rope_sin = burn::float_from_data(ctx, sn.data(), {c.max_ctx, D});
+    m->rope_cos = burn::float_from_data(ctx, cs.data(), {cap, D});
+    m->rope_sin = burn::float_from_data(ctx, sn.data(), {cap, D});
   } catch (const std::exception &e) {
     delete m;
     return fail_model(e);

@@ -390,3 +390,32 @@ def test_generate_rejects_zero_new_tokens(engine, smol):
     with pytest.raises(miburn.MiError) as e:
         m.generate(np.zeros((1, 4), np.int32), 0)
     assert e.value.kind == "ARG"
+
+
+@pytest.mark.parametrize("batch,t,longer,numerics", [(1, 300, 320, "reference"), (3, 100, 128, "reference"),
+                                                     (1, 17, 32, "performance"), (2, 33, 48, "performance")])
+def test_ragged_prompt_runs_padded(engine, batch, t, longer, numerics):
+    """A prompt off 32 rows runs on padding positions: its logits are bit for
+    bit the first positions' of the longer prompt that fills those rows, and
+    the positions after it see none of them (a step after the prompt, and one
+    at the last position the context holds)."""
+    cfg = dict(vocab=512, hidden=128, layers=2, heads=2, kv_heads=1, head_dim=64, intermediate=256,
+               rope_theta=10000.0, eps=1e-5)
+    ids = np.random.default_rng(t).integers(0, 512, (batch, longer + 2)).astype(np.int32)
+    m = miburn.Llama(engine, cfg, max_ctx=t + 2, max_batch=batch, seed=4, init_std=0.05, numerics=numerics)
+    full = miburn.Llama(engine, cfg, max_ctx=longer, max_batch=batch, seed=4, init_std=0.05, numerics=numerics)
+    got = engine.download(m.forward(ids[:, :t], all_positions=True)).reshape(batch, t, -1)
+    want = engine.download(full.forward(ids[:, :longer], all_positions=True)).reshape(batch, longer, -1)[:, :t]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    W = weights(engine, m, cfg)
+    ref = ref_logits(W, cfg, ids[:, :t + 2])
+    for i in range(2):
+        close_logits(engine.download(m.forward(ids[:, t + i:t + i + 1])), ref[:, t + i],
+                     2e-3 if numerics == "reference" else 2e-2)
+    with pytest.raises(miburn.MiError):  # the context is what was asked for, padding or not
+        m.forward(ids[:, :1])
+    out, _, _ = m.generate(ids[:, :t], 2)
+    traced, _, _ = m.generate(ids[:, :t], 2, traced=True)
+    assert np.array_equal(out, traced)
+    m.close()
+    full.close()
