@@ -34,6 +34,8 @@
 #include "gemm_args.hpp"
 #include "wave.hpp"
 
+#include <cmath>
+
 namespace mi {
 
 // Element types: uint16_t carries BF16 bits, float is F32.
@@ -2086,16 +2088,50 @@ static hipError_t pack_operand(hipStream_t st, const void *src, int elem, bool s
   return hipGetLastError();
 }
 
+// The tiles of a product of any shape: each k-tile of 32 takes about c us of a
+// CU (measured at one tile a CU; the operands' DMA from L2 bounds the smaller
+// ones, 50 GB/s a CU, the MFMAs the largest), and the busiest CU has
+// ceil(tiles / 256) of them.  us, packs included: 1500 x 3072 over k 1536, 288
+// tiles of 128 x 128 in two rounds 36.0, 192 of 192 x 128 in one 25.6; 3001 x
+// 2500 F32 over 3 x 2048, 480 of 128 x 128 140, 240 of 256 x 128 119; 4095 x
+// 4097 over 4001, 272 of 256 x 256 217, 726 of 192 x 128 200; 4000 x 2300 F32
+// over 3 x 1024, 288 of 192 x 128 95, 144 of 256 x 256 88.
+struct AnyTile {
+  int bm, bn;
+  double c;
+};
+static const AnyTile ANY_TILES[4] = {{128, 128, 0.33}, {192, 128, 0.41}, {256, 128, 0.50}, {256, 256, 0.83}};
+
+static int any_tile(const Plan &q) {
+  int best = 0;
+  double least = 0;
+  for (int t = 0; t < 4; ++t) {
+    const AnyTile &a = ANY_TILES[t];
+    const int64_t tiles = ((q.M + a.bm - 1) / a.bm) * ((q.N + a.bn - 1) / a.bn) * q.batch;
+    const double us = static_cast<double>((tiles + 255) / 256) * (q.K / 32 * a.c + 1.5);
+    if (t == 0 || us < least) {
+      best = t;
+      least = us;
+    }
+  }
+  return best;
+}
+
 template <typename TO, bool BKC>
 static hipError_t launch_any_tile(const Plan &q, hipStream_t st) {
-  const bool whole = !q.ka;  // the whole-tile form reads A's k as it lies
-  const int64_t t256 = ((q.M + 255) / 256) * ((q.N + 255) / 256) * q.batch;
-  if (t256 >= 192) {
-    if (whole && q.M % 256 == 0 && q.N % 256 == 0) return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 0>(q, st);
-    return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 2>(q, st);
+  const int t = any_tile(q);
+  // The whole-tile form reads A's k as it lies.
+  const bool whole = !q.ka && q.M % ANY_TILES[t].bm == 0 && q.N % ANY_TILES[t].bn == 0;
+  switch (t) {
+    case 0:
+      if (whole) return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 0>(q, st);
+      return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 2>(q, st);
+    case 1: return launch_pipe_cfg<TO, 192, 128, 5, true, BKC, 2, 2, 2>(q, st);
+    case 2: return launch_pipe_cfg<TO, 256, 128, 5, true, BKC, 4, 2, 2>(q, st);
+    default:
+      if (whole) return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 0>(q, st);
+      return launch_pipe_cfg<TO, 256, 256, 5, true, BKC, 2, 4, 2>(q, st);
   }
-  if (whole && q.M % 128 == 0 && q.N % 128 == 0) return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 0>(q, st);
-  return launch_pipe_cfg<TO, 128, 128, 5, true, BKC, 2, 2, 2>(q, st);
 }
 
 // The BF16 products that run_bf16 sends to the direct kernel as they lie.
@@ -2107,19 +2143,47 @@ static bool exactly_direct(const Plan &p) {
          ((p.M + 127) / 128) * ((p.N + 127) / 128) >= 128;
 }
 
+// Whether operand x of a product can be read by the direct kernel as it lies.
+static bool lies_for_dma(const Plan &p, const void *x, int64_t ld, int64_t item) {
+  return p.K % 32 == 0 && ld % 8 == 0 && item % 8 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15);
+}
+static bool a_in_place(const Plan &p) { return p.ea == MI_BF16 && !p.ta && lies_for_dma(p, p.a, p.lda, p.sa); }
+static bool b_in_place(const Plan &p) {
+  return p.eb == MI_BF16 && (p.tb || p.N % 8 == 0) && lies_for_dma(p, p.b, p.ldb, p.sb);
+}
+
+// A BF16 product off the whole tiles: the time of the guarded 64 x 64 tiles
+// (125 TF/s over a full chip of 16-byte chunks, 30 where the pitch puts rows
+// off them and every element is loaded by itself) against the direct kernel's
+// (450 TF/s) and its packs' (3 us and the bytes at 4 TB/s each); fewer tiles
+// than fill the chip cost either about the square root of what they leave
+// idle (split-K, the clock).
+static bool bf16_any_pays(const Plan &p, int64_t t128) {
+  const bool chunks = p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sa % 8 == 0 && p.sb % 8 == 0 &&
+                      !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15);
+  if (t128 < (chunks ? 32 : 8)) return false;
+  const double flop = 2.0 * static_cast<double>(p.M) * p.N * p.K * p.batch;
+  const double t64 = static_cast<double>(((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch);
+  const double guarded = flop / ((chunks ? 125e6 : 30e6) * std::min(1.0, std::sqrt(t64 / 1024)));
+  double direct = 1.5 + flop / (450e6 * std::min(1.0, std::sqrt(static_cast<double>(t128) / 256)));
+  if (!a_in_place(p)) direct += 3 + static_cast<double>(p.M * p.K * (p.sa ? p.batch : 1)) * 4 / 4e6;
+  if (!b_in_place(p)) direct += 3 + static_cast<double>(p.N * p.K * (p.sb ? p.batch : 1)) * 4 / 4e6;
+  return direct < guarded;
+}
+
 // Whether a product goes to the direct kernel through packed operands.  Both
 // sides of each line measured (us, this path after what ran before):
 //  * F32 x F32 in the fast mode, where it splits (2^33 multiply-adds, 128
 //    tiles; below that F32 products keep the F32 matrix cores' precision):
 //    4096^3 992 -> 372 (370 TF/s), 4095^3 1790 -> 384, 3001 x 2500 x 2047
-//    431 -> 140.  The split kernel converts every tile again for each block
+//    431 -> 120.  The split kernel converts every tile again for each block
 //    that reads it, with no k-tile in flight behind the one it multiplies.
 //  * F32 activations x BF16: 4000 x 4000 x 3000 674 -> 193, 1500 x 3072 x 768
-//    93 -> 42; 2000 x 576 x 1536 37.7 -> 40.0, below the line at 2^31.
-//  * BF16 off the whole tiles: 2001^3 450 -> 38.8, 4095 x 4097 x 4001 1719 ->
-//    215 (transposed A 5180 -> 217), 1000^3 42.6 -> 21.3, 700^3 29.2 -> 17.1;
-//    100 x 3000 x 1000 (24 tiles) 16.4 -> 20.9 and 512 x 512 x 500 (16 tiles)
-//    19.8 -> 12.7 lie below the line at 32 tiles.
+//    93 -> 31; 2000 x 576 x 1536 37.7 -> 40.0, below the line at 2^31.
+//  * BF16 off the whole tiles, by bf16_any_pays: 2001^3 450 -> 38.8, 4095 x
+//    4097 x 4001 1719 -> 200 (transposed A 5180 -> 202), 1000^3 42.6 -> 21.3,
+//    700^3 29.2 -> 17.1, 512 x 512 x 500 19.8 -> 12.7; 2134 x 1840 x 136 (8.7
+//    against 13.0) and 100 x 3000 x 1000 (16.4 against 20.9) stay.
 static bool direct_any_pays(const Plan &p) {
   if (p.per_group || p.kc || p.swiglu || p.qkv.mode || p.M < 16 || p.N < 16) return false;
   const bool f32 = p.ea == MI_F32 || p.eb == MI_F32;
@@ -2127,7 +2191,7 @@ static bool direct_any_pays(const Plan &p) {
   if (p.K >= (int64_t(1) << 24) || p.lda >= (int64_t(1) << 26) || p.ldb >= (int64_t(1) << 26)) return false;
   const int64_t macs = p.M * p.N * p.K * p.batch;
   const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-  if (!f32) return macs >= (int64_t(1) << 28) && t128 >= 32;
+  if (!f32) return bf16_any_pays(p, t128);
   if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return macs >= (int64_t(1) << 31) && t128 >= 128;
   return macs >= (int64_t(1) << 33) && t128 >= 128;
 }
@@ -2139,11 +2203,7 @@ static int run_direct_any(mi_ctx *ctx, const Plan &p, bool *ran) {
   Plan q = p;
   const int na = p.ea == MI_F32 ? 2 : 1, nb = p.eb == MI_F32 ? 2 : 1;
   const int64_t kp = (p.K + 31) / 32 * 32;
-  auto lies = [&](const void *x, int64_t ld, int64_t item) {
-    return p.K % 32 == 0 && ld % 8 == 0 && item % 8 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15);
-  };
-  const bool a_in = na == 1 && !p.ta && lies(p.a, p.lda, p.sa);
-  const bool b_in = nb == 1 && (p.tb || p.N % 8 == 0) && lies(p.b, p.ldb, p.sb);
+  const bool a_in = a_in_place(p), b_in = b_in_place(p);
   const int64_t ia = p.sa ? p.batch : 1, ib = p.sb ? p.batch : 1;
   const int64_t n8 = (p.N + 7) / 8 * 8;
   mi_id aid = 0, bid = 0;

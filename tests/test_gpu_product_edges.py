@@ -40,6 +40,10 @@ def test_bf16_split_k_of_a_half_k_tile(engine, m, n, k):
     (777, 2049, 257, False, False, "bf16"),    # odd pitch, one column past a tile
     (513, 1025, 640, True, False, "f32"),      # transposed A
     (3585, 3841, 96, True, True, "f32"),       # 256-row tiles, one past the last
+    (1501, 3065, 512, False, True, "f32"),     # 192 x 128 tiles
+    (1501, 3064, 500, False, False, "bf16"),
+    (3001, 2500, 512, False, True, "f32"),     # 256 x 128 tiles
+    (3001, 2497, 500, False, False, "f32"),
 ])
 def test_bf16_any_shape(engine, m, n, k, ta, tb, out):
     a, b = _ints((k, m) if ta else (m, k)), _ints((n, k) if tb else (k, n))
