@@ -162,3 +162,67 @@ def test_f32_sum_has_no_bias(engine):
     sd = d.std()
     assert abs(d.mean()) < 6 * sd / np.sqrt(m * n)                       # independent errors' mean
     assert np.abs(d.mean(axis=0)).max() < 7 * sd / np.sqrt(m)            # and each column's
+
+
+# ------------------------------------------------------ rows of any width
+WIDE_ROWS = [(3, 1025), (5, 2048), (7, 2049), (300, 4095), (2, 4097), (9, 8001), (4, 8192)]
+
+
+@pytest.mark.parametrize("rows,cols", WIDE_ROWS)
+def test_wide_row_norms(engine, rows, cols):
+    """RMSNorm and LayerNorm with a block a row, against float64: rel 1e-5."""
+    x = (RNG.standard_normal((rows, cols)) + 0.5).astype(np.float32)
+    g, b = RNG.standard_normal((1, cols)).astype(np.float32), RNG.standard_normal((1, cols)).astype(np.float32)
+    ids = [engine.upload(t) for t in (x, g, b)]
+    xd = x.astype(np.float64)
+    rms = xd / np.sqrt((xd * xd).mean(1, keepdims=True) + 1e-5)
+    c = xd - xd.mean(1, keepdims=True)
+    ln = c / np.sqrt((c * c).mean(1, keepdims=True) + 1e-5)
+    for o, want in ((engine.rms_norm(ids[0], ids[1]), rms * g), (engine.rms_norm(ids[0]), rms),
+                    (engine.layer_norm(ids[0], ids[1], ids[2]), ln * g + b), (engine.layer_norm(ids[0]), ln)):
+        got = engine.download(o)
+        engine.free(o)
+        assert np.abs(got - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+    for t in ids:
+        engine.free(t)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 512), (3, 515), (300, 2049), (5, 8001), (4097, 1023), (256, 1), (256, 33),
+                                       (64, 128), (257, 40), (7, 100000)])
+def test_row_and_column_folds(engine, rows, cols):
+    """Sums, maxima, minima and means over either axis, and a NaN in them."""
+    x = RNG.standard_normal((rows, cols)).astype(np.float32)
+    ix = engine.upload(x)
+    for axis, ax in ((miburn.AXIS_COLS, 1), (miburn.AXIS_ROWS, 0)):
+        n = x.shape[ax]
+        for op, f in ((miburn.R_SUM, np.sum), (miburn.R_MEAN, np.mean), (miburn.R_MAX, np.max), (miburn.R_MIN, np.min)):
+            o = engine.reduce(ix, op, axis)
+            got = engine.download(o).reshape(-1)
+            engine.free(o)
+            want = f(x.astype(np.float64), axis=ax)
+            if op in (miburn.R_MAX, miburn.R_MIN):
+                assert np.array_equal(got, want.astype(np.float32))
+            else:  # n roundings of 2^-24 of sum |x|
+                bound = n * 2.0 ** -24 * np.abs(x).astype(np.float64).sum(ax) / (n if op == miburn.R_MEAN else 1)
+                assert np.all(np.abs(got - want) <= bound + 1e-30)
+    engine.free(ix)
+    x[0, cols // 2] = np.nan
+    ix = engine.upload(x)
+    for op in (miburn.R_SUM, miburn.R_MAX, miburn.R_MIN):
+        o = engine.reduce(ix, op, miburn.AXIS_COLS)
+        got = engine.download(o).reshape(-1)
+        engine.free(o)
+        assert np.isnan(got[0]) and not np.isnan(got[1:]).any()
+    engine.free(ix)
+
+
+@pytest.mark.parametrize("n", [1, 64, 2048, 2049])
+def test_whole_folds(engine, n):
+    x = RNG.standard_normal((1, n)).astype(np.float32)
+    ix = engine.upload(x)
+    for op, f in ((miburn.R_SUM, np.sum), (miburn.R_MEAN, np.mean), (miburn.R_MAX, np.max)):
+        o = engine.reduce_all(ix, op)
+        got = float(engine.download(o)[0, 0])
+        engine.free(o)
+        assert abs(got - f(x.astype(np.float64))) <= n * 2.0 ** -24 * max(1e-3, np.abs(x).sum() / (n if f is np.mean else 1))
+    engine.free(ix)
