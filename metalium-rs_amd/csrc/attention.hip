@@ -1329,7 +1329,7 @@ int attention_plan(Ctx *ctx, mi_id q, mi_id k_cache, mi_id v_cache, int64_t batc
   P->kv16 = kb->elem == MI_BF16;
   P->D = D; P->G = G; P->maxc = maxc; P->items = items; P->S = S; P->chunk = chunk;
   // The matrix-core kernel for 64+ new positions with 64-wide heads, its
-  // keys split into ranges on small grids (whole, paired runs of a 512-token
+  // keys split into ranges on small grids (whole runs of a 512-token
   // prompt at batch 1 took 4.27 ms against 3.92 on the key-chunked kernel).
   P->flash = !pos_dev && span == pos0 + t && D == 64 && t >= FLASH_MIN_T && batch * kv_heads <= 65535;
   P->fchunk = P->fS = 0;

@@ -771,6 +771,28 @@ __global__ void __launch_bounds__(256) softmax_long_kernel(const void *x, int el
 }
 
 // ------------------------------------------------------- RMSNorm, LayerNorm
+// Column j of a row's result in the form asked for.
+__device__ __forceinline__ void norm_put(void *out, int out_elem, int64_t row, int64_t rows, int64_t j, int64_t cols,
+                                         float y) {
+  if (out_elem == MI_BF16_PARTS) {
+    uint16_t h, l;
+    split_bf16(y, h, l);
+    uint16_t *o = static_cast<uint16_t *>(out) + 2 * row * cols;
+    o[j] = h;
+    o[cols + j] = l;
+  } else if (out_elem == MI_TILES_PARTS) {
+    uint16_t h, l;
+    split_bf16(y, h, l);
+    uint16_t *o = static_cast<uint16_t *>(out) + tile_offset(row, j, cols);
+    o[0] = h;
+    o[rows * cols] = l;
+  } else if (out_elem == MI_TILES_BF16) {
+    static_cast<uint16_t *>(out)[tile_offset(row, j, cols)] = f32_to_bf16_bits(y);
+  } else {
+    st(out, out_elem, row * cols + j, y);
+  }
+}
+
 // XF: the input and the gain F32, fixed at compile time (else read from elem
 // and gelem); OE >= 0: the result's form, fixed likewise.  The fixed forms
 // carry no element switch around each load and store.
@@ -812,23 +834,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *x, int elem, 
       } else {
         if (gamma) y = y * ld(gamma, gelem, j);
       }
-      if (out_elem == MI_BF16_PARTS) {
-        uint16_t h, l;
-        split_bf16(y, h, l);
-        uint16_t *o = static_cast<uint16_t *>(out) + 2 * base;
-        o[j] = h;
-        o[cols + j] = l;
-      } else if (out_elem == MI_TILES_PARTS) {
-        uint16_t h, l;
-        split_bf16(y, h, l);
-        uint16_t *o = static_cast<uint16_t *>(out) + tile_offset(row, j, cols);
-        o[0] = h;
-        o[rows * cols] = l;
-      } else if (out_elem == MI_TILES_BF16) {
-        static_cast<uint16_t *>(out)[tile_offset(row, j, cols)] = f32_to_bf16_bits(y);
-      } else {
-        st(out, out_elem, base + j, y);
-      }
+      norm_put(out, out_elem, row, rows, j, cols, y);
     }
   }
 }
@@ -891,7 +897,7 @@ __global__ void __launch_bounds__(256) layer_norm_kernel(const float *x, const f
 // -> 7.8.
 template <int NTH, bool LN>
 __global__ void __launch_bounds__(NTH) norm_block_kernel(const float *x, const float *gamma, const float *beta, float eps,
-                                                         float *out, int64_t cols) {
+                                                         void *out_any, int out_elem, int64_t cols) {
   constexpr int NW = NTH / 64;
   __shared__ float red[2][NW];
   const int tid = threadIdx.x;
@@ -951,23 +957,25 @@ __global__ void __launch_bounds__(NTH) norm_block_kernel(const float *x, const f
       if (LN && beta) t = t + b[u][e];
       y[e] = t;
     }
-    if (c + 4 <= cols) {
+    float *out = static_cast<float *>(out_any);
+    if (out_elem == MI_F32 && c + 4 <= cols) {
       *reinterpret_cast<f32x4u *>(out + base + c) = y;
     } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < cols) out[base + c + e] = y[e];
+      for (int e = 0; e < 4 && c + e < cols; ++e) {
+        if (LN || out_elem == MI_F32) out[base + c + e] = y[e];
+        else norm_put(out_any, out_elem, blockIdx.x, gridDim.x, c + e, cols, y[e]);
+      }
     }
   }
 }
 
 template <bool LN>
-static void norm_block_launch(Ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, float *out,
-                              int64_t R, int64_t C) {
+static void norm_block_launch(Ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, void *out,
+                              int out_elem, int64_t R, int64_t C) {
   const unsigned g = static_cast<unsigned>(R);
-  if (C <= 2048) norm_block_kernel<256, LN><<<g, 256, 0, ctx->stream>>>(x, gamma, beta, eps, out, C);
-  else if (C <= 4096) norm_block_kernel<512, LN><<<g, 512, 0, ctx->stream>>>(x, gamma, beta, eps, out, C);
-  else norm_block_kernel<1024, LN><<<g, 1024, 0, ctx->stream>>>(x, gamma, beta, eps, out, C);
+  if (C <= 2048) norm_block_kernel<256, LN><<<g, 256, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
+  else if (C <= 4096) norm_block_kernel<512, LN><<<g, 512, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
+  else norm_block_kernel<1024, LN><<<g, 1024, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
 }
 
 // Register-row kernels: the smallest T (columns per lane) covering `cols`.
@@ -1166,9 +1174,9 @@ void rms_norm_launch(Ctx *ctx, const void *xp, int xe, const void *gp, int ge, f
                      int64_t R, int64_t C) {
   // Wide F32 rows a block each (up to 2048 columns a wavefront a row keeps
   // the split-K reduce's bits, splitk_reduce_norm).
-  if (xe == MI_F32 && (gp == nullptr || ge == MI_F32) && out_elem == MI_F32 && C > 2048 && R <= INT32_MAX) {
-    norm_block_launch<false>(ctx, static_cast<const float *>(xp), static_cast<const float *>(gp), nullptr, eps,
-                             static_cast<float *>(out), R, C);
+  if (xe == MI_F32 && (gp == nullptr || ge == MI_F32) && C > 2048 && R <= INT32_MAX) {
+    norm_block_launch<false>(ctx, static_cast<const float *>(xp), static_cast<const float *>(gp), nullptr, eps, out,
+                             out_elem, R, C);
     return;
   }
   // One wavefront a row; below 4096 rows one a block, so the rows spread
@@ -1261,7 +1269,7 @@ extern "C" int mi_layer_norm(mi_ctx *ctx, mi_id a, mi_id gamma, mi_id beta, floa
   int s = new_buffer(ctx, R, C, MI_F32, &id, &ob);
   if (s) return s;
   if (R > 0 && C > 1024 && R <= INT32_MAX) {
-    norm_block_launch<true>(ctx, xp, gp, bp, eps, static_cast<float *>(ob->ptr), R, C);
+    norm_block_launch<true>(ctx, xp, gp, bp, eps, ob->ptr, MI_F32, R, C);
   } else if (R > 0 && C > 0) {
     unsigned g = grid_for(R, 4, INT32_MAX);
     float *o = static_cast<float *>(ob->ptr);
