@@ -309,7 +309,8 @@ int mi_linear_qkv_rope_cache(mi_ctx *ctx, mi_id x, int x_parts, mi_id w_qkv,
  *   |a||b| (the reference's fast mode rounds operands to TF32, 2^-11).  Other
  *   products run as in ACCURATE.  A non-finite operand element gives NaN in
  *   its row or column where F32 arithmetic could give an infinity.
- *  ACCURATE: F32 products on the F32 matrix cores, F32 accumulation.
+ *  ACCURATE: F32 products at F32 precision, F32 accumulation: on the F32 matrix
+ *   cores, or on the BF16 ones with each element in three parts (24 bits).
  * The reference's EXACT mode (k-ordered sequential F32 sums) is not offered:
  * MI_E_UNSUPPORTED. ---- */
 enum mi_matmul_mode { MI_MATMUL_FAST = 0, MI_MATMUL_ACCURATE = 1 };

@@ -18,10 +18,11 @@
 //    stages: one's barrier and epilogue under the other's products.
 //
 // us, against the register-staged 64 x 64 / 128 x 128 kernel it replaces:
-// 4096^3 (accurate mode) 1090 -> 762 (180 TF/s), 2048 x 8192 x 256 82 -> 59,
-// [256, 8192] over k 2000 transposed 137 -> 72, 16 x 512^3 44.0 -> 30.8, 1500^3
-// 127 -> 64, 512^3 15.2 -> 9.5, 64 x 128 x 784 12.5 -> 9.7.  The error against
-// float64 falls at each (4096^3 1.15e-6 -> 1.0e-6, 1500^3 6.9e-7 -> 3.4e-7).
+// 4096^3 (accurate mode) 1075 -> 809 (170 TF/s; 762 at best), 2048 x 8192 x 256
+// 82 -> 63, [256, 8192] over k 2000 transposed 138 -> 71, 16 x 512^3 44.0 ->
+// 33.9, 1500^3 128 -> 65, 512^3 15.0 -> 9.6, 64 x 128 x 784 12.4 -> 9.5.  The
+// error against float64 falls at each (4096^3 1.1e-6 -> 1.0e-6, 1500^3 6.9e-7
+// -> 3.4e-7).
 //
 // LDS tiles.  An operand whose k is contiguous lies as 128-byte rows of 32 k
 // in 16-byte chunks, chunk c of row r at c ^ (r / 2 & 7); a lane's fragment is one
@@ -325,7 +326,7 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
     // a result's rows or columns (a bias gradient) would collect.  Odd rows of
     // A and odd columns of B are taken with their sign turned, so results of
     // either parity lean either way (sum over 2000 rows of a [2000, 8192] x
-    // [8192, 256] product: error 1.7e-6 without, 6e-7 with).
+    // [8192, 256] product: error 1.7e-6 without, at most 4.5e-7 with).
     const uint32_t sg = static_cast<uint32_t>(lane & 1) << 31;
     Raw8 raw[2][TF];
     Parts3 part[2][TF];
