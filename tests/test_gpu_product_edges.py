@@ -226,3 +226,26 @@ def test_whole_folds(engine, n):
         engine.free(o)
         assert abs(got - f(x.astype(np.float64))) <= n * 2.0 ** -24 * max(1e-3, np.abs(x).sum() / (n if f is np.mean else 1))
     engine.free(ix)
+
+
+# Products over a long k with few tiles are summed in slices: the error of one
+# F32 chain of n = k / 16 matrix-core steps is a random walk of roundings of
+# partial sums that grow as sqrt(i), 0.4 * 2^-24 * sqrt(n / 2) of the result,
+# and slices stay below it (1.0e-7 at the first; one chain reaches 2.2e-7).
+@pytest.mark.parametrize("m,n,k,ta,tb", [
+    (1656, 372, 1415, False, True),
+    (777, 777, 3001, False, False),
+    (300, 300, 3001, False, True),
+])
+def test_bf16_long_k_keeps_its_slices(engine, m, n, k, ta, tb):
+    rng = np.random.default_rng(k)
+    a = bf16_to_f32(bf16_bits(rng.standard_normal((k, m) if ta else (m, k), dtype=np.float32)))
+    b = bf16_to_f32(bf16_bits(rng.standard_normal((n, k) if tb else (k, n), dtype=np.float32)))
+    ia, ib = engine.upload_bf16(bf16_bits(a)), engine.upload_bf16(bf16_bits(b))
+    o = engine.matmul_dram(ia, ta, ib, tb, miburn.F32)
+    got = engine.download(o).astype(np.float64).reshape(m, n)
+    for i in (ia, ib, o):
+        engine.free(i)
+    want = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err < 0.4 * 2.0 ** -24 * np.sqrt(k / 32)
