@@ -245,15 +245,24 @@ Tensor forward_rows(mi_llama *m, Tensor x, int64_t batch, int64_t t);
 // (sequence, position)), before the final norm.
 Tensor forward_ids(mi_llama *m, const Tensor &idx, int64_t batch, int64_t t) {
   const int64_t hid = m->cfg.hidden, pos0 = m->len, tp = padded_positions(m, batch, t, pos0);
-  Tensor x = burn::select_rows_as(m->embed, idx, MI_F32);  // [rows, hidden], the BF16 rows widened
-  x = x.reshape({batch * t, hid});
-  if (tp == t) return forward_rows(m, x, batch, t);
-  const int64_t dims[4] = {1, batch, t, hid}, real[4] = {0, t * hid, hid, 1}, pad[4] = {0, tp * hid, hid, 1};
-  Tensor xp = burn::fill(m->ctx, {batch * tp, hid}, MI_F32, 0);
-  burn::copy_into4(xp, 0, pad, x, 0, real, dims);
-  x = forward_rows(m, xp, batch, tp);
+  Tensor ids = idx;
+  if (tp != t) {
+    // The padding repeats each sequence's last token: rows like its own, so
+    // finite where they are (a row of zeros is 0 / 0 in an RMSNorm of eps 0,
+    // and its NaN values reach real queries through the masked keys' 0 * NaN).
+    const int64_t src[4] = {0, 0, t, 1}, last[4] = {0, 0, t, 0}, dst[4] = {0, 0, tp, 1};
+    const int64_t real[4] = {1, 1, batch, t}, pad[4] = {1, 1, batch, tp - t};
+    ids = burn::empty(m->ctx, {batch * tp}, MI_I32);
+    burn::copy_into4(ids, 0, dst, idx, 0, src, real);
+    burn::copy_into4(ids, t, dst, idx, t - 1, last, pad);
+  }
+  Tensor x = burn::select_rows_as(m->embed, ids, MI_F32);  // [rows, hidden], the BF16 rows widened
+  x = x.reshape({batch * tp, hid});
+  x = forward_rows(m, x, batch, tp);
+  if (tp == t) return x;
   m->len = pos0 + t;
-  return burn::copy4(x, dims, 0, pad).reshape({batch * t, hid});
+  const int64_t rows[4] = {1, batch, t, hid}, st[4] = {0, tp * hid, hid, 1};
+  return burn::copy4(x, rows, 0, st).reshape({batch * t, hid});
 }
 
 // The forward of the embedded rows x [batch * t, hidden] at the cache's length.

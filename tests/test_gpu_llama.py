@@ -419,3 +419,17 @@ def test_ragged_prompt_runs_padded(engine, batch, t, longer, numerics):
     assert np.array_equal(out, traced)
     m.close()
     full.close()
+
+
+@pytest.mark.parametrize("batch,t,numerics", [(1, 300, "reference"), (3, 100, "reference"), (1, 17, "performance"),
+                                              (2, 33, "performance")])
+def test_ragged_prompt_without_eps(engine, batch, t, numerics):
+    """eps 0: the padding rows of a ragged prompt are finite, so its last
+    positions, whose key block they share, are what the CPU model gives."""
+    cfg = dict(vocab=512, hidden=128, layers=2, heads=2, kv_heads=1, head_dim=64, intermediate=256,
+               rope_theta=10000.0, eps=0.0)
+    ids = np.random.default_rng(t).integers(0, 512, (batch, t)).astype(np.int32)
+    m = miburn.Llama(engine, cfg, max_ctx=t, max_batch=batch, seed=4, init_std=0.05, numerics=numerics)
+    got = engine.download(m.forward(ids, all_positions=True)).reshape(batch, t, -1)
+    close_logits(got, ref_logits(weights(engine, m, cfg), cfg, ids), 2e-3 if numerics == "reference" else 2e-2)
+    m.close()
