@@ -678,7 +678,7 @@ log_softmax_ce_kernel(const float *z, const int32_t *tgt, int64_t cols, float gs
   for (int t = 0; t < T; ++t) {
     const int64_t j = col_of(t);
     v[t] = v[t] - ls;  // logp_j
-    if (j == target) picked[row] = v[t];
+    if (j == target && in_range) picked[row] = v[t];  // a thread's columns run past the row
     v[t] = __fadd_rn(j == target ? -gscale : 0.0f, __fmul_rn(expf(v[t]), gscale));
   }
   if constexpr (VEC) {
@@ -726,7 +726,8 @@ __global__ void __launch_bounds__(256) log_softmax_ce_wave_kernel(const float *z
   s = wave_sum(s);
   const float ls = logf(s);
   const int32_t target = tgt[row];
-  if (lane == 0 && !(target >= 0 && target < cols)) {
+  const bool in_range = target >= 0 && target < cols;
+  if (lane == 0 && !in_range) {
     atomicOr(flags, FLAG_INDEX_RANGE);
     picked[row] = 0.0f;
   }
@@ -734,7 +735,7 @@ __global__ void __launch_bounds__(256) log_softmax_ce_wave_kernel(const float *z
   for (int t = 0; t < T; ++t) {
     const int64_t j = lane + 64 * t;
     const float lp = v[t] - ls;
-    if (j == target) picked[row] = lp;
+    if (j == target && in_range) picked[row] = lp;  // a lane's columns run past the row
     if (j < cols) dz[base + j] = __fadd_rn(j == target ? -gscale : 0.0f, __fmul_rn(expf(lp), gscale));
   }
 }

@@ -560,6 +560,22 @@ def test_log_softmax_ce_target_out_of_range_is_domain(engine):
     assert p[1, 0] == 0.0 and p[3, 0] == 0.0
 
 
+@pytest.mark.parametrize("cols,target", [(10, 12), (10, 63), (1001, 1020), (1500, 1900), (3000, 4090), (3001, 4000)])
+def test_log_softmax_ce_target_past_the_row_picks_nothing(engine, cols, target):
+    """A target past the row and within its threads' last columns: picked 0
+    and no one-hot term, as for any target out of range."""
+    engine.sync()
+    z = rnd(3, cols)
+    iz, it = engine.upload(z), engine.upload_i32(np.array([[1], [target], [cols - 1]], np.int32))
+    ip, idz = engine.log_softmax_ce(iz, it, 0.25)
+    with pytest.raises(miburn.MiError) as e:
+        engine.sync()
+    assert e.value.kind == "DOMAIN"
+    p, dz = engine.download(ip), engine.download(idz)
+    assert p[1, 0] == 0.0 and (p[[0, 2], 0] < 0).all()
+    assert abs(dz[1].sum() - 0.25) < 1e-5  # the softmax row times 0.25
+
+
 # --------------------------------------------- split-K slices folded by SGD
 @pytest.mark.parametrize("m,n,k,ta,sliced", [(256, 256, 2048, True, True), (1024, 256, 2048, True, True),
                                              (256, 768, 2048, True, True), (64, 128, 784, False, True),
