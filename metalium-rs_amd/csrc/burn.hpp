@@ -18,6 +18,13 @@
 
 #include "../../include/miburn.h"
 
+namespace mi {
+// mi_log_softmax_ce with the gradient's rule for a target out of range
+// (csrc/reduce.hip).
+int log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float grad_scale, bool drop_lost, mi_id *picked,
+                   mi_id *dlogits);
+}  // namespace mi
+
 namespace burn {
 
 struct Error : std::runtime_error {
@@ -223,13 +230,16 @@ inline Tensor float_matmul(const Tensor &a, bool ta, const Tensor &b, bool tb, i
 
 // Cross-entropy against integer targets and its gradient in one pass:
 // picked = logp at each row's target ([rows, 1]), dlogits = exp(logp) * s
-// minus s at the target.
+// minus s at the target.  drop_lost: zero in a row whose target is out of
+// range, as log_softmax's backward composed op by op gives (mi_log_softmax_ce
+// leaves exp(logp) * s there).
 struct CrossEntropy {
   Tensor picked, dlogits;
 };
-inline CrossEntropy log_softmax_ce(const Tensor &logits, const Tensor &targets, float grad_scale) {
+inline CrossEntropy log_softmax_ce(const Tensor &logits, const Tensor &targets, float grad_scale,
+                                   bool drop_lost = false) {
   mi_id p, d;
-  check(logits.ctx(), mi_log_softmax_ce(logits.ctx(), logits.use(), targets.use(), grad_scale, &p, &d),
+  check(logits.ctx(), mi::log_softmax_ce(logits.ctx(), logits.use(), targets.use(), grad_scale, drop_lost, &p, &d),
         "log_softmax_ce");
   return {Tensor(logits.ctx(), p, {logits.rows(), 1}), Tensor(logits.ctx(), d, {logits.rows(), logits.cols()})};
 }

@@ -58,11 +58,11 @@ Tensor step(mi_mlp *m, const Tensor &x, const Tensor &labels, float lr) {
   Tensor h = burn::relu(burn::linear(x, m->w1, false, &m->b1, nullptr));
   Tensor z = burn::linear(h, m->w2, false, &m->b2, nullptr);
   // Cross-entropy and its gradient: in one pass over the logits (the bits of
-  // the composition; with the bias epilogues and slices 100 -> 63 us a step at
+  // the composition, also where a label is out of range; with the bias epilogues and slices 100 -> 63 us a step at
   // batch 64, a launch each 3-5 us of it), or composed where the rows are longer than that pass takes.
   Tensor loss, dz;
   if (m->d_out <= 16384) {
-    burn::CrossEntropy ce = burn::log_softmax_ce(z, labels, 1.0f / static_cast<float>(B));
+    burn::CrossEntropy ce = burn::log_softmax_ce(z, labels, 1.0f / static_cast<float>(B), true);
     loss = burn::float_neg(burn::reduce_all(ce.picked, MI_R_MEAN));  // [1, 1]
     dz = ce.dlogits;
   } else {

@@ -614,15 +614,17 @@ softmax_row_kernel(const float *x, float scale, float *out) {
 // picked[row], and dz_j = e^(logp_j) * gscale + (j == t ? -gscale : 0) -- the
 // same two roundings as exp, then MUL_ADD against the scattered one-hot --
 // written to dz.  A target outside [0, cols) raises the index flag, picks 0
-// bits and adds no one-hot term (as pick_columns and scatter_add_columns).
+// bits and adds no one-hot term (as pick_columns and scatter_add_columns);
+// with drop_lost its row's gradient is zero, as log-softmax's own backward
+// forms it (g - exp(logp) sum(g), g the scattered one-hot: nothing there).
 // NTH threads a row: thread t holds float4 lanes t + NTH u (VEC) or values
 // t + NTH u, folded as the softmax kernel that runs the log-softmax of the
 // same row folds (softmax_row_kernel, NTH = columns / 8, for rows of 2048,
 // 4096 or 8192 columns; softmax_block_kernel, NTH = 256, otherwise).
 template <int VPT, bool VEC, bool NT, int NTH = 256>
 __global__ void __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(VPT <= 8 ? 8 : 4)))
-log_softmax_ce_kernel(const float *z, const int32_t *tgt, int64_t cols, float gscale, float *picked, float *dz,
-                      uint32_t *flags) {
+log_softmax_ce_kernel(const float *z, const int32_t *tgt, int64_t cols, float gscale, bool drop_lost, float *picked,
+                      float *dz, uint32_t *flags) {
   constexpr int T = 4 * VPT, NW = NTH / 64;
   __shared__ float red[2][NW];
   const int64_t row = blockIdx.x;
@@ -674,6 +676,7 @@ log_softmax_ce_kernel(const float *z, const int32_t *tgt, int64_t cols, float gs
     atomicOr(flags, FLAG_INDEX_RANGE);
     picked[row] = 0.0f;
   }
+  if (drop_lost && !in_range) gscale = 0.0f;
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const int64_t j = col_of(t);
@@ -700,8 +703,8 @@ log_softmax_ce_kernel(const float *z, const int32_t *tgt, int64_t cols, float gs
 // holds columns l + 64 t), in the order of the wavefront softmax.
 template <int T>
 __global__ void __launch_bounds__(256) log_softmax_ce_wave_kernel(const float *z, const int32_t *tgt, int64_t rows,
-                                                                  int64_t cols, float gscale, float *picked, float *dz,
-                                                                  uint32_t *flags) {
+                                                                  int64_t cols, float gscale, bool drop_lost, float *picked,
+                                                                  float *dz, uint32_t *flags) {
   const int lane = threadIdx.x & 63;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -731,6 +734,7 @@ __global__ void __launch_bounds__(256) log_softmax_ce_wave_kernel(const float *z
     atomicOr(flags, FLAG_INDEX_RANGE);
     picked[row] = 0.0f;
   }
+  if (drop_lost && !in_range) gscale = 0.0f;
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const int64_t j = lane + 64 * t;
@@ -1447,8 +1451,9 @@ extern "C" int mi_layer_norm_backward(mi_ctx *ctx, mi_id x, mi_id gamma, mi_id d
   return MI_OK;
 }
 
-extern "C" int mi_log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float grad_scale, mi_id *picked,
-                                 mi_id *dlogits) {
+namespace mi {
+int log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float grad_scale, bool drop_lost, mi_id *picked,
+                   mi_id *dlogits) {
   MI_ENTER(ctx);
   if (!picked || !dlogits) return fail(ctx, MI_E_ARG, "null out pointer");
   MI_BUF(ctx, zb, logits);
@@ -1472,7 +1477,7 @@ extern "C" int mi_log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float
     // The row lengths the log-softmax runs a wavefront per row on.
     const unsigned g = grid_for(R, 4, INT32_MAX);
     switch (pick_t(C)) {
-#define MI_CEW(T) case T: log_softmax_ce_wave_kernel<T><<<g, 256, 0, ctx->stream>>>(zp, tp, R, C, grad_scale, pp, dp, flags(ctx)); break;
+#define MI_CEW(T) case T: log_softmax_ce_wave_kernel<T><<<g, 256, 0, ctx->stream>>>(zp, tp, R, C, grad_scale, drop_lost, pp, dp, flags(ctx)); break;
       MI_CEW(1) MI_CEW(2) MI_CEW(4) MI_CEW(8) MI_CEW(16)
 #undef MI_CEW
     }
@@ -1487,16 +1492,16 @@ extern "C" int mi_log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float
     // Rows of 2048, 4096 or 8192: the layout of softmax_row_kernel.
     if (C == 1024 * vpt && vpt >= 2 && vpt <= 8) {
       switch (vpt * 2 + (nt ? 1 : 0)) {
-#define MI_CER(V) case 2 * V: log_softmax_ce_kernel<2, true, false, 128 * V><<<g, 128 * V, 0, ctx->stream>>>(zp, tp, C, grad_scale, pp, dp, flags(ctx)); break; \
-                  case 2 * V + 1: log_softmax_ce_kernel<2, true, true, 128 * V><<<g, 128 * V, 0, ctx->stream>>>(zp, tp, C, grad_scale, pp, dp, flags(ctx)); break;
+#define MI_CER(V) case 2 * V: log_softmax_ce_kernel<2, true, false, 128 * V><<<g, 128 * V, 0, ctx->stream>>>(zp, tp, C, grad_scale, drop_lost, pp, dp, flags(ctx)); break; \
+                  case 2 * V + 1: log_softmax_ce_kernel<2, true, true, 128 * V><<<g, 128 * V, 0, ctx->stream>>>(zp, tp, C, grad_scale, drop_lost, pp, dp, flags(ctx)); break;
         MI_CER(2) MI_CER(4) MI_CER(8)
 #undef MI_CER
       }
     } else
     switch (vpt) {
-#define MI_CE(V) case V: if (nt) log_softmax_ce_kernel<V, true, true><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, pp, dp, flags(ctx)); \
-                         else if (vec) log_softmax_ce_kernel<V, true, false><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, pp, dp, flags(ctx)); \
-                         else log_softmax_ce_kernel<V, false, false><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, pp, dp, flags(ctx)); break;
+#define MI_CE(V) case V: if (nt) log_softmax_ce_kernel<V, true, true><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, drop_lost, pp, dp, flags(ctx)); \
+                         else if (vec) log_softmax_ce_kernel<V, true, false><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, drop_lost, pp, dp, flags(ctx)); \
+                         else log_softmax_ce_kernel<V, false, false><<<g, 256, 0, ctx->stream>>>(zp, tp, C, grad_scale, drop_lost, pp, dp, flags(ctx)); break;
       MI_CE(1) MI_CE(2) MI_CE(4) MI_CE(8) MI_CE(16)
 #undef MI_CE
     }
@@ -1506,6 +1511,12 @@ extern "C" int mi_log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float
   *picked = pid;
   *dlogits = did;
   return MI_OK;
+}
+}  // namespace mi
+
+extern "C" int mi_log_softmax_ce(mi_ctx *ctx, mi_id logits, mi_id targets, float grad_scale, mi_id *picked,
+                                 mi_id *dlogits) {
+  return mi::log_softmax_ce(ctx, logits, targets, grad_scale, false, picked, dlogits);
 }
 
 extern "C" int mi_softmax_backward(mi_ctx *ctx, mi_id p, mi_id dp, float scale, mi_id *out) {

@@ -73,3 +73,33 @@ def test_config1_loss_falls(engine):
     # SGD from the init must move it down from where it started.
     assert losses[:10].mean() > losses[-10:].mean()
     assert ms > 0
+
+
+@pytest.mark.parametrize("d_out", [10, 1500, 17000])  # a wavefront a row, a block a row, the composed step
+def test_label_out_of_range_has_no_gradient(engine, d_out):
+    """The step's labels out of range are DOMAIN at the next wait; their rows
+    add nothing to the loss's sum and nothing to any gradient."""
+    engine.sync()
+    d_in, hid, B, lr = 20, 8, 4, 0.5
+    m = miburn.Mlp(engine, d_in, hid, d_out)
+    rng = np.random.default_rng(2)
+    x, y = rng.random((B, d_in), dtype=np.float32), np.array([1, d_out + 2, d_out - 1, -1], np.int32)
+    params = [torch.tensor(p, dtype=torch.float64, requires_grad=True) for p in lcg_init(d_in, hid, d_out)]
+    w1, b1, w2, b2 = params
+    z = torch.relu(torch.from_numpy(x).double() @ w1 + b1) @ w2 + b2
+    loss = -torch.log_softmax(z, 1)[[0, 2], [1, d_out - 1]].sum() / B
+    loss.backward()
+    ids = engine.upload(x), engine.upload_i32(y.reshape(-1, 1))
+    got = m.train_step_ids(*ids, lr)
+    with pytest.raises(miburn.MiError) as e:
+        engine.sync()
+    assert e.value.kind == "DOMAIN"
+    assert abs(engine.download(got)[0, 0] - loss.item()) <= 1e-5 * loss.item()
+    for i, p in enumerate(params):
+        step = lcg_init(d_in, hid, d_out)[i] - m.param(i)
+        want = lr * p.grad.numpy()
+        # Each parameter's own rounding, and F32 sums.
+        assert np.abs(step - want).max() <= 2.0 ** -23 * np.abs(p.detach().numpy()).max() + 1e-5 * np.abs(want).max()
+    for t in (*ids, got):
+        engine.free(t)
+    m.close()
