@@ -2261,10 +2261,18 @@ static int run_direct_any(mi_ctx *ctx, const Plan &p, bool *ran) {
   return check_launch(ctx, "matmul");
 }
 
+// Whether run_product takes the product through packed operands.
+static bool packed_direct(const Plan &p) { return direct_any_pays(p) && !exactly_direct(p); }
+
+// The split-K slices of the product as run_product runs it (1: none).
+static int product_slices(const Plan &p) {
+  return stacked_split_pays(p) || packed_direct(p) || gemv_fits(p) ? 1 : splitk_slices(p);
+}
+
 static int run_product(mi_ctx *ctx, Plan &p) {
   hipError_t e;
   if (stacked_split_pays(p)) return run_stacked_split(ctx, p);
-  if (direct_any_pays(p) && !exactly_direct(p)) {
+  if (packed_direct(p)) {
     bool ran;
     const int s = run_direct_any(ctx, p, &ran);
     if (s || ran) return s;
@@ -2450,7 +2458,7 @@ extern "C" int mi_matmul_slices(mi_ctx *ctx, mi_id a, int a_transposed, mi_id b,
                 (long long)p.K, (long long)kb, (long long)p.N);
   p.batch = 1; p.sa = p.sb = p.sc = 0;
   p.lda = A->cols; p.ldb = B->cols;
-  p.splits = (p.M > 0 && p.N > 0 && p.K > 0 && !gemv_fits(p)) ? splitk_slices(p) : 1;
+  p.splits = (p.M > 0 && p.N > 0 && p.K > 0) ? product_slices(p) : 1;
   if (p.splits <= 1) {
     *slices = 1;
     return matmul_common(ctx, a, a_transposed, b, b_transposed, 1, 0, 0, 0, 0, nullptr, MI_F32, out);

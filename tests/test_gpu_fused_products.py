@@ -595,6 +595,29 @@ def test_matmul_slices_sum_to_the_product(engine, m, n, k, ta, sliced):
     assert (S > 1) == sliced
 
 
+@pytest.mark.parametrize("mode", [miburn.MATMUL_FAST, miburn.MATMUL_ACCURATE])
+@pytest.mark.parametrize("m,n,k,ta", [(2048, 1024, 8192, True), (1536, 1536, 8192, True), (1500, 1500, 4096, True),
+                                      (2000, 1408, 4096, False)])
+def test_matmul_slices_of_large_products(engine, m, n, k, ta, mode):
+    """Past the fast mode's line too, the slices sum to the product's bits:
+    one slice where the product runs whole on BF16 parts."""
+    engine.set_matmul_mode(mode)
+    try:
+        ia, ib = engine.upload(rnd(k, m) if ta else rnd(m, k)), engine.upload(rnd(k, n))
+        sid, S = engine.matmul_slices(ia, ta, ib, False)
+        parts = engine.download(sid)
+        total = parts[:m].copy()
+        for z in range(1, S):
+            total = (total + parts[z * m:(z + 1) * m]).astype(np.float32)
+        o = engine.matmul_dram(ia, ta, ib, False)
+        same_bits(total, engine.download(o))
+        assert mode != miburn.MATMUL_FAST or S == 1
+        for t in (ia, ib, sid, o):
+            engine.free(t)
+    finally:
+        engine.set_matmul_mode(miburn.MATMUL_FAST)
+
+
 def test_sgd_folds_stacked_slices(engine):
     lr = np.float32(0.05)
     # A weight gradient from slices, against the same update from the reduced product.
