@@ -2269,6 +2269,14 @@ static int product_slices(const Plan &p) {
   return stacked_split_pays(p) || packed_direct(p) || gemv_fits(p) ? 1 : splitk_slices(p);
 }
 
+// The slices' partial products of a product that splits over k (p.splits set),
+// or null: one that does not, or whose scratch cannot be had, runs whole.
+static float *splitk_scratch(mi_ctx *ctx, Plan &p) {
+  p.splits = splitk_slices(p);
+  if (p.splits <= 1) return nullptr;
+  return static_cast<float *>(scratch(ctx, static_cast<size_t>(p.splits) * p.M * p.N * sizeof(float)));
+}
+
 static int run_product(mi_ctx *ctx, Plan &p) {
   hipError_t e;
   if (stacked_split_pays(p)) return run_stacked_split(ctx, p);
@@ -2280,9 +2288,7 @@ static int run_product(mi_ctx *ctx, Plan &p) {
   if (gemv_fits(p)) {
     launch_gemv(p, ctx->stream);
     e = hipGetLastError();
-  } else if ((p.splits = splitk_slices(p)) > 1) {
-    float *part = static_cast<float *>(scratch(ctx, static_cast<size_t>(p.splits) * p.M * p.N * sizeof(float)));
-    if (!part) return fail(ctx, MI_E_OOM, "split-K scratch");
+  } else if (float *part = splitk_scratch(ctx, p)) {
     e = run_splitk(p, part, ctx->stream);
   } else {
     p.splits = 1;
