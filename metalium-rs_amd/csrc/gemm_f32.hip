@@ -12,10 +12,11 @@
 //    chain of latencies.
 //  * 64 x 128 and 128 x 128 on v_mfma_f32_32x32x16_bf16: each value, read from
 //    LDS, is split in registers into three BF16 parts (24 bits in all) and a
-//    product taken as the six part products above 2^-24 of it: 6 x 32 cycles
-//    for 16 k against 512.  The 15 vector operations a pair of values run
-//    between the MFMAs of the step before.  Two blocks a CU, each two LDS
-//    stages: one's barrier and epilogue under the other's products.
+//    product taken as six of the nine part products, the others at most 2^-24
+//    of it together: 6 x 32 cycles for 16 k against 512.  The 13 vector
+//    operations a pair of values run between the MFMAs of the step before.  Two
+//    blocks a CU, each two LDS stages: one's barrier and epilogue under the
+//    other's products.
 //
 // us, against the register-staged 64 x 64 / 128 x 128 kernel it replaces:
 // 4096^3 (accurate mode) 1075 -> 809 (170 TF/s; 762 at best), 2048 x 8192 x 256
@@ -136,21 +137,19 @@ struct F32Operand {
   }
 };
 
-// Two F32 values as three BF16 parts each, packed in pairs: the value rounded
-// to 8 bits (half up in magnitude), the remainder's leading 8 bits, and the at
-// most 8 that are left, 24 bits in all.  The rounded head leaves a remainder
-// of either sign, so the parts' products that are left out (middle times
-// remainder, 2^-25 of a product and less) cancel over a sum.  The values are
-// taken with their sign turned where sg is 0x80000000.
+// Two F32 values as three BF16 parts each, packed in pairs: each part the
+// nearest BF16 of what the ones before leave.  The head leaves at most 2^-8 of
+// the value, in 16 bits, the middle at most 2^-17, in 7, so the three hold its
+// 24 bits, and the part products that are left out (middle times remainder and
+// less) come to at most 2^-24 of a product, of either sign.  The values are
+// taken with their sign turned where sg is 0x80000000. 
 __device__ __forceinline__ void split3_pair(float x, float y, uint32_t sg, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
   const float a = __uint_as_float(__float_as_uint(x) ^ sg), b = __uint_as_float(__float_as_uint(y) ^ sg);
-  const uint32_t ha = __float_as_uint(a) + 0x8000u, hb = __float_as_uint(b) + 0x8000u;
-  hi = __builtin_amdgcn_perm(hb, ha, 0x07060302u);
-  const float ra = a - __uint_as_float(ha & 0xffff0000u), rb = b - __uint_as_float(hb & 0xffff0000u);
-  mid = __builtin_amdgcn_perm(__float_as_uint(rb), __float_as_uint(ra), 0x07060302u);
-  const float la = ra - __uint_as_float(__float_as_uint(ra) & 0xffff0000u);
-  const float lb = rb - __uint_as_float(__float_as_uint(rb) & 0xffff0000u);
-  lo = __builtin_amdgcn_perm(__float_as_uint(lb), __float_as_uint(la), 0x07060302u);
+  hi = bf16x2_bits(a, b);
+  const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xffff0000u);
+  mid = bf16x2_bits(ra, rb);
+  const float la = ra - __uint_as_float(mid << 16), lb = rb - __uint_as_float(mid & 0xffff0000u);
+  lo = bf16x2_bits(la, lb);
 }
 
 struct Raw8 {  // a lane's eight k of one fragment
@@ -371,8 +370,8 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
                   __builtin_bit_cast(bf16x8, part[st][i].p[PA[t]]),
                   __builtin_bit_cast(bf16x8, part[st][TM + j].p[PB[t]]), accs[st % NA][i][j], 0, 0, 0);
             }
-            // The step's 15 operations a pair of values spread over its MFMAs.
-            spread<0, MF, (60 * TF + MF - 1) / MF>();
+            // The step's 13 operations a pair of values spread over its MFMAs.
+            spread<0, MF, (52 * TF + MF - 1) / MF>();
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -527,8 +526,13 @@ static double f32_time(const Plan &p, const F32Tile &t, int64_t S) {
 }
 
 // The best tile for S slices.  4-byte DMA leaves no registers for the largest.
+// Sums of up to 32 products stay on the F32 matrix cores, where an outer
+// product is one rounding (4096 x 1 x 4096: 2.5e-8 from float64 against 3.5e-8
+// from parts); 4096 x 4096 over k 16 and 32 23.0 and 20.6 us against 27.1 and
+// 20.9 on 128 x 128.
 static int f32_tile(const Plan &p, int64_t S) {
   int best = 0;
+  if (p.K <= 32) return best;
   for (int t = 1; t < (f32_quads(p) ? 3 : 2); ++t)
     if (f32_time(p, F32_TILES[t], S) < f32_time(p, F32_TILES[best], S)) best = t;
   return best;

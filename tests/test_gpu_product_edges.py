@@ -249,3 +249,16 @@ def test_bf16_long_k_keeps_its_slices(engine, m, n, k, ta, tb):
     want = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err < 0.4 * 2.0 ** -24 * np.sqrt(k / 32)
+
+
+@pytest.mark.parametrize("m,n", [(4096, 4096), (2047, 2049)])
+@pytest.mark.parametrize("k", [1, 2, 8, 33])
+def test_f32_short_k_is_f32_arithmetic(engine, m, n, k):
+    """Sums of few products over results large enough for any tile: an outer
+    product is one rounding of each product, 2^-24 of it, and k products at
+    most k of sum |a||b| (each product's and each sum's but the first)."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    got = _f32_product(engine, a, False, b, False)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b)) * (1 + 2.0 ** -20))
