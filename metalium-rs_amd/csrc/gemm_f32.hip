@@ -13,7 +13,7 @@
 //  * 64 x 128 and 128 x 128 on v_mfma_f32_32x32x16_bf16: each value, read from
 //    LDS, is split in registers into three BF16 parts (24 bits in all) and a
 //    product taken as six of the nine part products, the others at most 2^-24
-//    of it together: 6 x 32 cycles for 16 k against 512.  The 13 vector
+//    of it together: 6 x 32 cycles for 16 k against 512.  The 14 vector
 //    operations a pair of values run between the MFMAs of the step before.  Two
 //    blocks a CU, each two LDS stages: one's barrier and epilogue under the
 //    other's products.
@@ -142,14 +142,20 @@ struct F32Operand {
 // the value, in 16 bits, the middle at most 2^-17, in 7, so the three hold its
 // 24 bits, and the part products that are left out (middle times remainder and
 // less) come to at most 2^-24 of a product, of either sign.  The values are
-// taken with their sign turned where sg is 0x80000000. 
-__device__ __forceinline__ void split3_pair(float x, float y, uint32_t sg, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+// taken with their sign turned where sg is 0x80000000.  A value below about
+// 2^-110 leaves bits under BF16's least subnormal, 2^-133: the low halves of
+// its remainder's word, collected in lost.
+__device__ __forceinline__ void split3_pair(float x, float y, uint32_t sg, uint32_t &hi, uint32_t &mid, uint32_t &lo,
+                                            uint32_t &lost) {
   const float a = __uint_as_float(__float_as_uint(x) ^ sg), b = __uint_as_float(__float_as_uint(y) ^ sg);
   hi = bf16x2_bits(a, b);
   const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xffff0000u);
   mid = bf16x2_bits(ra, rb);
   const float la = ra - __uint_as_float(mid << 16), lb = rb - __uint_as_float(mid & 0xffff0000u);
   lo = bf16x2_bits(la, lb);
+  // (In asm, or the compiler keeps every remainder to collect them as a tree:
+  // 48 spilled registers on 128 x 128.)
+  asm("v_or3_b32 %0, %1, %2, %0" : "+v"(lost) : "v"(la), "v"(lb));
 }
 
 struct Raw8 {  // a lane's eight k of one fragment
@@ -165,11 +171,11 @@ __device__ __forceinline__ float at4(const float4 &v, int e) {
 __device__ __forceinline__ float raw_at(const Raw8 &r, int e) { return at4(e < 4 ? r.a : r.b, e & 3); }
 
 // Pair q (0 .. 3) of a fragment's eight values into its parts.
-__device__ __forceinline__ void split_piece(const Raw8 &r, Parts3 &o, int q, uint32_t sg) {
-  if (q == 0) split3_pair(r.a.x, r.a.y, sg, o.p[0].x, o.p[1].x, o.p[2].x);
-  else if (q == 1) split3_pair(r.a.z, r.a.w, sg, o.p[0].y, o.p[1].y, o.p[2].y);
-  else if (q == 2) split3_pair(r.b.x, r.b.y, sg, o.p[0].z, o.p[1].z, o.p[2].z);
-  else split3_pair(r.b.z, r.b.w, sg, o.p[0].w, o.p[1].w, o.p[2].w);
+__device__ __forceinline__ void split_piece(const Raw8 &r, Parts3 &o, int q, uint32_t sg, uint32_t &lost) {
+  if (q == 0) split3_pair(r.a.x, r.a.y, sg, o.p[0].x, o.p[1].x, o.p[2].x, lost);
+  else if (q == 1) split3_pair(r.a.z, r.a.w, sg, o.p[0].y, o.p[1].y, o.p[2].y, lost);
+  else if (q == 2) split3_pair(r.b.x, r.b.y, sg, o.p[0].z, o.p[1].z, o.p[2].z, lost);
+  else split3_pair(r.b.z, r.b.w, sg, o.p[0].w, o.p[1].w, o.p[2].w, lost);
 }
 
 // At most M DMA instructions (63 where M is more: the counter's range) and no
@@ -318,7 +324,7 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
     fold_accs();
   } else {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) load(s, s);
+    for (int s = 0; s < NS; ++s) load(s < ktiles ? s : 0, s);
     // Step 0's parts and step 1's values of the first tile.
     // An MFMA drops, downward, the bits of a small product that lie below its
     // accumulator's last: a bias of 2^-8 of a rounding, but one that a sum over
@@ -329,6 +335,9 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
     const uint32_t sg = static_cast<uint32_t>(lane & 1) << 31;
     Raw8 raw[2][TF];
     Parts3 part[2][TF];
+    // Bits that the parts could not hold.  The last tile splits its other stage
+    // once more, which holds the tile before it or (one tile) the tile itself.
+    uint32_t lost = 0;
     static_assert(NS == 2, "the waits below");
     if (ktiles > 1) wait_tile<PER_TILE>();
     else wait_tile<0>();
@@ -339,7 +348,7 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
 #pragma unroll
     for (int f = 0; f < TF; ++f)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) split_piece(raw[0][f], part[0][f], q, sg);
+      for (int q = 0; q < 4; ++q) split_piece(raw[0][f], part[0][f], q, sg, lost);
 
     // Tile kt + s multiplies the parts at hand; its own stage is free (its
     // values were read a tile ago) and takes tile kt + s + NS, while the next
@@ -362,7 +371,7 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
             __builtin_amdgcn_sched_barrier(0);
             constexpr int MF = 6 * TM * TN;
 #pragma unroll
-            for (int q = 0; q < 4 * TF; ++q) split_piece(raw[st ^ 1][q / 4], part[st ^ 1][q / 4], q % 4, sg);
+            for (int q = 0; q < 4 * TF; ++q) split_piece(raw[st ^ 1][q / 4], part[st ^ 1][q / 4], q % 4, sg, lost);
 #pragma unroll
             for (int q = 0; q < MF; ++q) {
               const int t = q / (TM * TN), i = q % (TM * TN) / TN, j = q % TN;
@@ -370,8 +379,8 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
                   __builtin_bit_cast(bf16x8, part[st][i].p[PA[t]]),
                   __builtin_bit_cast(bf16x8, part[st][TM + j].p[PB[t]]), accs[st % NA][i][j], 0, 0, 0);
             }
-            // The step's 13 operations a pair of values spread over its MFMAs.
-            spread<0, MF, (52 * TF + MF - 1) / MF>();
+            // The step's 14 operations a pair of values spread over its MFMAs.
+            spread<0, MF, (56 * TF + MF - 1) / MF>();
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -389,8 +398,10 @@ __global__ void __launch_bounds__(WM *WN * 64, 2) gemm_f32_kernel(GemmArgs g) {
 
     // A result that is not finite came from an operand that is not, or from a
     // head rounded up to infinity: the parts of such a value are not F32
-    // arithmetic on it, so the tile is formed again on the F32 matrix cores.
-    uint32_t bad = 0;
+    // arithmetic on it, nor are those of a value too small for three, so the
+    // tile is formed again on the F32 matrix cores (4096^3 737 us; with such a
+    // value in every tile 1693).
+    uint32_t bad = lost & 0xffffu;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll

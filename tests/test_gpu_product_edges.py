@@ -110,7 +110,7 @@ def test_f32_any_shape_bias_residual(engine):
 # whole and with edges, each DMA width, k-tile remainders, one k-tile, slices.
 F32_SHAPES = [(64, 64, 32), (64, 64, 8), (65, 67, 33), (1, 1, 1), (130, 66, 20), (128, 192, 96), (512, 512, 512),
               (2048, 768, 256), (2050, 772, 260), (2049, 771, 259), (2048, 2048, 64), (2052, 2044, 68),
-              (257, 129, 2047), (1500, 1500, 300)]
+              (257, 129, 2047), (1500, 1500, 300), (2048, 2048, 512)]
 
 
 def _f32_product(engine, a, ta, b, tb):
@@ -262,3 +262,33 @@ def test_f32_short_k_is_f32_arithmetic(engine, m, n, k):
     got = _f32_product(engine, a, False, b, False)
     want = a.astype(np.float64) @ b.astype(np.float64)
     assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b)) * (1 + 2.0 ** -20))
+
+
+# 64 x 128 and 128 x 128 tiles, whole, with edges and by 4-byte DMA, and slices.
+@pytest.mark.parametrize("m,n,k", [(2048, 768, 256), (2048, 2048, 512), (1500, 1500, 300), (2049, 771, 259),
+                                   (256, 512, 2065)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+@pytest.mark.parametrize("small", ["a", "b", "a few"])
+def test_f32_small_operands(engine, m, n, k, ta, tb, small):
+    """Values whose last bits lie below BF16's least subnormal (2^-133), down to
+    F32's own subnormals, against ones that bring their products to ordinary
+    size: an F32 sum's bound, as for any other values."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.standard_normal((m, k)), rng.standard_normal((k, n))
+    if small == "a few":  # one column of A below, its row of B far above the rest
+        a[:, 5] = np.ldexp(a[:, 5], -118)
+        b[5] = np.ldexp(b[5], 118)
+    else:
+        e = rng.integers(-130, -108, (1, k))
+        a, b = (np.ldexp(a, e), np.ldexp(b, 110)) if small == "a" else (np.ldexp(a, 110), np.ldexp(b, e.T))
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    got = _f32_product(engine, a.T.copy() if ta else a, ta, b.T.copy() if tb else b, tb)
+    av, bv = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(got - av @ bv) <= (k + 4) * 2.0 ** -24 * (np.abs(av) @ np.abs(bv)))
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 512), (1500, 1500, 300), (2048, 768, 256), (2049, 771, 259)])
+def test_f32_non_finite_operands_on_every_parts_tile(engine, m, n, k):
+    """As test_f32_non_finite_operands, on 128 x 128 tiles whole and with edges,
+    64 x 128 ones, and by 4-byte DMA."""
+    test_f32_non_finite_operands(engine, m, n, k)
