@@ -498,17 +498,24 @@ static hipError_t launch_f32_orient(const Plan &p, hipStream_t st) {
   return launch_f32<BM, BN, WM, WN, NS, SPLIT, false, false, EDGE>(p, st);
 }
 
-bool f32_pipe_fits(const Plan &p) {
-  // A lane's byte offset in a tile is 32 bits: 128 rows of the pitch.
-  return p.ea == MI_F32 && p.eb == MI_F32 && p.lda < (int64_t(1) << 22) && p.ldb < (int64_t(1) << 22);
-}
-
 // Sixteen-byte DMA: pitches, item strides, pointers and contiguous extents in
 // fours (split-K slices start on k-tiles).
 static bool f32_quads(const Plan &p) {
   return p.lda % 4 == 0 && p.ldb % 4 == 0 && p.sa % 4 == 0 && p.sb % 4 == 0 && p.sa2 % 4 == 0 && p.sb2 % 4 == 0 &&
          !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15) &&
          (p.ta ? p.M : p.K) % 4 == 0 && (p.tb ? p.K : p.N) % 4 == 0;
+}
+
+bool f32_pipe_fits(const Plan &p) {
+  // Operands by 4-byte DMA over k up to 8 (one with its k contiguous): a k-tile
+  // of 32 is mostly lanes past k, and the register-staged kernel, which loads
+  // them not at all, sums in the same order.  us there / here: 4096 x 4096 x 1
+  // 23.1 / 30.2, x 2 with B^T 23.2 / 30.5; over k 9 to 63 it is still ahead (k 9
+  // 24.8 / 30.6) by up to a quarter, but one chain over k errs more (k 16
+  // 7.4e-8 against 6.0e-8).
+  if (p.K <= 8 && !f32_quads(p) && (!p.ta || p.tb)) return false;
+  // A lane's byte offset in a tile is 32 bits: 128 rows of the pitch.
+  return p.ea == MI_F32 && p.eb == MI_F32 && p.lda < (int64_t(1) << 22) && p.ldb < (int64_t(1) << 22);
 }
 
 // The tiles: 64 x 64 on the F32 matrix cores, 64 x 128 and 128 x 128 on BF16

@@ -252,7 +252,7 @@ def test_bf16_long_k_keeps_its_slices(engine, m, n, k, ta, tb):
 
 
 @pytest.mark.parametrize("m,n", [(4096, 4096), (2047, 2049)])
-@pytest.mark.parametrize("k", [1, 2, 8, 33])
+@pytest.mark.parametrize("k", [1, 2, 7, 8, 9, 33])
 def test_f32_short_k_is_f32_arithmetic(engine, m, n, k):
     """Sums of few products over results large enough for any tile: an outer
     product is one rounding of each product, 2^-24 of it, and k products at
