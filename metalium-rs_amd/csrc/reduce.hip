@@ -974,12 +974,19 @@ __global__ void __launch_bounds__(NTH) norm_block_kernel(const float *x, const f
   }
 }
 
+// Whether a launch holds R blocks of nth threads: past 2^32 threads it runs the
+// first of them only, with no error.
+static bool grid_holds(int64_t R, int nth) { return R < (int64_t(1) << 32) / nth; }
+// norm_block_kernel's threads a row of C columns.
+static int norm_block_threads(int64_t C) { return C <= 2048 ? 256 : C <= 4096 ? 512 : 1024; }
+
 template <bool LN>
 static void norm_block_launch(Ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, void *out,
                               int out_elem, int64_t R, int64_t C) {
   const unsigned g = static_cast<unsigned>(R);
-  if (C <= 2048) norm_block_kernel<256, LN><<<g, 256, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
-  else if (C <= 4096) norm_block_kernel<512, LN><<<g, 512, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
+  const int nth = norm_block_threads(C);
+  if (nth == 256) norm_block_kernel<256, LN><<<g, 256, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
+  else if (nth == 512) norm_block_kernel<512, LN><<<g, 512, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
   else norm_block_kernel<1024, LN><<<g, 1024, 0, ctx->stream>>>(x, gamma, beta, eps, out, out_elem, C);
 }
 
@@ -1014,7 +1021,7 @@ extern "C" int mi_reduce(mi_ctx *ctx, mi_id a, int op, int axis, mi_id *out) {
   if (axis == MI_AXIS_COLS) {
     if (R > 0) {
       if (C == 0) fill_zero(ctx, o, R * sizeof(float));
-      else if (xe == MI_F32 && C >= 512 && R <= INT32_MAX && (R < 4096 || C % 4))
+      else if (xe == MI_F32 && C >= 512 && grid_holds(R, 256) && (R < 4096 || C % 4))
         reduce_cols_block_kernel<<<static_cast<unsigned>(R), 256, 0, ctx->stream>>>(static_cast<const float *>(xp), o, C, op);
       else if (R * C * 4 >= kStreamBytes)
         reduce_cols_kernel<true><<<grid_for(R, 4, INT32_MAX), 256, 0, ctx->stream>>>(xp, xe, o, R, C, op);
@@ -1179,7 +1186,7 @@ void rms_norm_launch(Ctx *ctx, const void *xp, int xe, const void *gp, int ge, f
                      int64_t R, int64_t C) {
   // Wide F32 rows a block each (up to 2048 columns a wavefront a row keeps
   // the split-K reduce's bits, splitk_reduce_norm).
-  if (xe == MI_F32 && (gp == nullptr || ge == MI_F32) && C > 2048 && R <= INT32_MAX) {
+  if (xe == MI_F32 && (gp == nullptr || ge == MI_F32) && C > 2048 && grid_holds(R, norm_block_threads(C))) {
     norm_block_launch<false>(ctx, static_cast<const float *>(xp), static_cast<const float *>(gp), nullptr, eps, out,
                              out_elem, R, C);
     return;
@@ -1273,7 +1280,7 @@ extern "C" int mi_layer_norm(mi_ctx *ctx, mi_id a, mi_id gamma, mi_id beta, floa
   mi_id id; Buffer *ob;
   int s = new_buffer(ctx, R, C, MI_F32, &id, &ob);
   if (s) return s;
-  if (R > 0 && C > 1024 && R <= INT32_MAX) {
+  if (R > 0 && C > 1024 && grid_holds(R, norm_block_threads(C))) {
     norm_block_launch<true>(ctx, xp, gp, bp, eps, ob->ptr, MI_F32, R, C);
   } else if (R > 0 && C > 0) {
     unsigned g = grid_for(R, 4, INT32_MAX);

@@ -292,3 +292,36 @@ def test_f32_non_finite_operands_on_every_parts_tile(engine, m, n, k):
     """As test_f32_non_finite_operands, on 128 x 128 tiles whole and with edges,
     64 x 128 ones, and by 4-byte DMA."""
     test_f32_non_finite_operands(engine, m, n, k)
+
+
+# ----------------------------------------------- more rows than one launch
+# A launch holds fewer than 2^32 threads: rows past those that a block each
+# fills it with.
+@pytest.fixture
+def own_engine():
+    with miburn.Engine(0) as eng:  # its tens of GB are given back with it
+        yield eng
+
+
+def test_reduce_of_2_24_rows(own_engine):
+    rows, cols = (1 << 24) + 3, 515
+    x = own_engine.fill(rows, cols, miburn.F32, int(np.float32(1.0).view(np.uint32)))
+    own_engine.assign_block(x, own_engine.upload(_ints((2, cols))), rows - 2, 0)
+    tail = own_engine.download(own_engine.copy_strided(x, 2, cols, (rows - 2) * cols, cols, 1))
+    got = own_engine.download(own_engine.reduce(x, miburn.R_SUM, miburn.AXIS_COLS)).reshape(-1)
+    assert np.all(got[:-2] == cols) and np.array_equal(got[-2:], tail.sum(1))
+
+
+@pytest.mark.parametrize("op,rows,cols", [("rms", (1 << 22) + 32, 4112), ("layer", (1 << 24) + 1, 1026)])
+def test_norms_of_many_wide_rows(own_engine, op, rows, cols):
+    x = own_engine.fill(rows, cols, miburn.F32, int(np.float32(2.0).view(np.uint32)))
+    last = RNG.standard_normal((1, cols)).astype(np.float32)
+    own_engine.assign_block(x, own_engine.upload(last), rows - 1, 0)
+    if op == "rms":
+        y, want = own_engine.rms_norm(x, 0, 0.0, miburn.BF16), last / np.sqrt((last.astype(np.float64) ** 2).mean())
+    else:
+        y, want = own_engine.layer_norm(x), (last - last.mean()) / np.sqrt(last.astype(np.float64).var() + 1e-5)
+    got = own_engine.download(own_engine.copy_strided(y, 3, cols, (rows - 3) * cols, cols, 1))
+    got = bf16_to_f32(got) if op == "rms" else got
+    assert np.array_equal(got[:2], np.full((2, cols), 1.0 if op == "rms" else 0.0))
+    assert np.abs(got[2] - want).max() <= (2.0 ** -8 if op == "rms" else 1e-5) * np.abs(want).max()
