@@ -39,59 +39,65 @@ __device__ __forceinline__ void st(void *p, int elem, int64_t i, float v) {
 }
 
 // ------------------------------------------------ reduce over columns (dim 1)
-// One wavefront per row; four rows per 256-thread block.
-template <bool NT>
-__global__ void __launch_bounds__(256) reduce_cols_kernel(const void *x, int elem, float *out, int64_t rows,
-                                                          int64_t cols, int op) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int64_t base = row * cols;
-  float acc = (op == MI_R_MAX) ? -INFINITY : (op == MI_R_MIN ? INFINITY : 0.0f);
-  if (elem == MI_F32 && (cols % 4) == 0) {
-    const float *p = static_cast<const float *>(x) + base;
-    const int64_t n4 = cols / 4;
-    auto fold = [op](float a, float4 v) {
-      if (op == MI_R_MAX) return max_nan(max_nan(max_nan(max_nan(a, v.x), v.y), v.z), v.w);
-      if (op == MI_R_MIN) return min_nan(min_nan(min_nan(min_nan(a, v.x), v.y), v.z), v.w);
-      return a + ((v.x + v.y) + (v.z + v.w));
-    };
-    int64_t j = lane;
-    // Four float4 per lane in flight, streamed when the input is large.
-    for (; j + 192 < n4; j += 256) {
-      float4 v0, v1, v2, v3;
-      if (NT) { v0 = ld4<true>(p + 4 * j); v1 = ld4<true>(p + 4 * (j + 64)); v2 = ld4<true>(p + 4 * (j + 128)); v3 = ld4<true>(p + 4 * (j + 192)); }
-      else { v0 = ld4<false>(p + 4 * j); v1 = ld4<false>(p + 4 * (j + 64)); v2 = ld4<false>(p + 4 * (j + 128)); v3 = ld4<false>(p + 4 * (j + 192)); }
-      acc = fold(fold(fold(fold(acc, v0), v1), v2), v3);
-    }
-    for (; j < n4; j += 64) acc = fold(acc, ld4<false>(p + 4 * j));
-  } else {
-    for (int64_t j = lane; j < cols; j += 64) {
-      float v = ld(x, elem, base + j);
-      if (op == MI_R_MAX) acc = max_nan(acc, v);
-      else if (op == MI_R_MIN) acc = min_nan(acc, v);
-      else acc += v;
-    }
-  }
-  if (op == MI_R_MAX) acc = wave_max(acc);
-  else if (op == MI_R_MIN) acc = wave_min(acc);
-  else acc = wave_sum(acc);
-  if (lane == 0) out[row] = (op == MI_R_MEAN) ? acc / static_cast<float>(cols) : acc;
-}
-
-// Four floats at any element alignment.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 // The fold of a reduction over `op`: NaN ranks above every number in a
 // maximum and below none in a minimum (max_nan, min_nan).
 __device__ __forceinline__ float fold_op(int op, float a, float b) {
   return op == MI_R_MAX ? max_nan(a, b) : op == MI_R_MIN ? min_nan(a, b) : a + b;
 }
 
-// F32 rows of any width and alignment, a 256-thread block a row: for rows too
-// few to fill the chip a wavefront each, and rows that 16-byte loads do not
-// divide (read as unaligned quads here, the last columns one by one).  300 x
-// 8001 20.8 -> 5.2 us, 3001 x 2049 12.5 -> 5.5, 8191 x 4095 27.8 -> 21.6.
+// One wavefront per row; four rows per 256-thread block.  Four chains a lane,
+// each over every fourth load: as many loads in flight, and sums of a quarter
+// the length.  The op is fixed at compile time: tested in the loop, the chains
+// ran twice as long as one (512 x 8192 2.0, now 0.91 of one chain's 4.9 us;
+// 16384 x 513 9.3 -> 5.6, 8191 x 4095 27.2 -> 20.5).
+template <bool NT, int op>
+__global__ void __launch_bounds__(256) reduce_cols_kernel(const void *x, int elem, float *out, int64_t rows,
+                                                          int64_t cols) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int64_t base = row * cols;
+  const float none = (op == MI_R_MAX) ? -INFINITY : (op == MI_R_MIN ? INFINITY : 0.0f);
+  float acc[4] = {none, none, none, none};
+  int64_t j = lane;
+  if (elem == MI_F32 && (cols % 4) == 0) {
+    const float *p = static_cast<const float *>(x) + base;
+    const int64_t n4 = cols / 4;
+    auto fold = [](float a, float4 v) { return fold_op(op, a, fold_op(op, fold_op(op, v.x, v.y), fold_op(op, v.z, v.w))); };
+    for (; j + 192 < n4; j += 256) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = ld4<NT>(p + 4 * (j + 64 * u));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] = fold(acc[u], v[u]);
+    }
+    for (; j < n4; j += 64) acc[0] = fold(acc[0], ld4<false>(p + 4 * j));
+  } else {
+    for (; j + 192 < cols; j += 256) {
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = ld(x, elem, base + j + 64 * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] = fold_op(op, acc[u], v[u]);
+    }
+    for (; j < cols; j += 64) acc[0] = fold_op(op, acc[0], ld(x, elem, base + j));
+  }
+  float r = fold_op(op, fold_op(op, acc[0], acc[1]), fold_op(op, acc[2], acc[3]));
+  r = op == MI_R_MAX ? wave_max(r) : op == MI_R_MIN ? wave_min(r) : wave_sum(r);
+  if (lane == 0) out[row] = (op == MI_R_MEAN) ? r / static_cast<float>(cols) : r;
+}
+
+// Four floats at any element alignment.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// F32 rows of any width and alignment, a 256-thread block a row, read as
+// unaligned quads (the last columns one by one).  For rows of 2000 columns and
+// more that 16-byte loads do not divide, where they are too few to fill the
+// chip with a wavefront each (up to 3072, or any number of 24576 columns) or
+// the input streams through (32768 rows).  us, a wavefront a row / this: 1000 x
+// 4095 7.5 / 4.2, 2048 x 8001 16.2 / 12.1, 512 x 30001 47.8 / 14.3, 65536 x 2047
+// 103 / 90; but 4096 x 3001 1.14 times as long, 16384 x 513 5.6 / 13.7, 1536 x
+// 8192 6.5 / 10.5.
 __global__ void __launch_bounds__(256) reduce_cols_block_kernel(const float *x, float *out, int64_t cols, int op) {
   __shared__ float red[4];
   const int tid = threadIdx.x;
@@ -1021,12 +1027,16 @@ extern "C" int mi_reduce(mi_ctx *ctx, mi_id a, int op, int axis, mi_id *out) {
   if (axis == MI_AXIS_COLS) {
     if (R > 0) {
       if (C == 0) fill_zero(ctx, o, R * sizeof(float));
-      else if (xe == MI_F32 && C >= 512 && grid_holds(R, 256) && (R < 4096 || C % 4))
+      else if (xe == MI_F32 && C % 4 && C >= 2000 && (R <= 3072 || R >= 32768 || C >= 24576) && grid_holds(R, 256))
         reduce_cols_block_kernel<<<static_cast<unsigned>(R), 256, 0, ctx->stream>>>(static_cast<const float *>(xp), o, C, op);
-      else if (R * C * 4 >= kStreamBytes)
-        reduce_cols_kernel<true><<<grid_for(R, 4, INT32_MAX), 256, 0, ctx->stream>>>(xp, xe, o, R, C, op);
       else
-        reduce_cols_kernel<false><<<grid_for(R, 4, INT32_MAX), 256, 0, ctx->stream>>>(xp, xe, o, R, C, op);
+        switch (op * 2 + (R * C * 4 >= kStreamBytes)) {
+#define MI_RC(OP)                                                                                                   \
+  case 2 * OP: reduce_cols_kernel<false, OP><<<grid_for(R, 4, INT32_MAX), 256, 0, ctx->stream>>>(xp, xe, o, R, C); break; \
+  case 2 * OP + 1: reduce_cols_kernel<true, OP><<<grid_for(R, 4, INT32_MAX), 256, 0, ctx->stream>>>(xp, xe, o, R, C); break;
+          MI_RC(MI_R_SUM) MI_RC(MI_R_MAX) MI_RC(MI_R_MEAN) MI_RC(MI_R_MIN)
+#undef MI_RC
+        }
     }
   } else if (C > 0) {
     if (R == 0) {
