@@ -804,6 +804,22 @@ __device__ __forceinline__ void norm_put(void *out, int out_elem, int64_t row, i
   }
 }
 
+// Columns c .. c + 3 of a row's result (c and cols multiples of 4) in any form
+// but F32: norm_put's values, 8 bytes a store.
+__device__ __forceinline__ void norm_put4(void *out, int out_elem, int64_t row, int64_t rows, int64_t c, int64_t cols,
+                                          float4 y) {
+  uint16_t *o = static_cast<uint16_t *>(out);
+  if (out_elem == MI_BF16_PARTS) {
+    o += 2 * row * cols + c;
+    parts4_put(o, o + cols, y);
+  } else if (out_elem == MI_TILES_PARTS) {
+    o += tile_offset(row, c, cols);
+    parts4_put(o, o + rows * cols, y);
+  } else {
+    f32x4_put(o + (out_elem == MI_TILES_BF16 ? tile_offset(row, c, cols) : row * cols + c), y);
+  }
+}
+
 // XF: the input and the gain F32, fixed at compile time (else read from elem
 // and gelem); OE >= 0: the result's form, fixed likewise.  The fixed forms
 // carry no element switch around each load and store.
@@ -906,13 +922,22 @@ __global__ void __launch_bounds__(256) layer_norm_kernel(const float *x, const f
 // gain read again after the fold.  us: RMSNorm 8192 x 4096 124 -> 40 (6.7 TB/s),
 // 8191 x 4095 125 -> 48, 300 x 8001 67 -> 6.1; LayerNorm 96 -> 42, 95 -> 56, 39
 // -> 7.8.
+// The other result forms, a wavefront a row / two bytes a store / eight, tiles
+// by XCD: 8192 x 4096 BF16 122 / 36 / 31, parts 140 / 51 / 40, tiles 125 / 84 /
+// 33, tiled parts 145 / 182 / 50.
 template <int NTH, bool LN>
 __global__ void __launch_bounds__(NTH) norm_block_kernel(const float *x, const float *gamma, const float *beta, float eps,
                                                          void *out_any, int out_elem, int64_t cols) {
   constexpr int NW = NTH / 64;
   __shared__ float red[2][NW];
   const int tid = threadIdx.x;
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * cols;
+  // A row in tiles is 16-byte pieces among those of the 31 beside it: the rows
+  // of a tile run on one XCD (workgroup w runs on XCD w % 8), whose L2 joins
+  // them before they are written.
+  int64_t row = blockIdx.x;
+  if (!LN && (out_elem == MI_TILES_BF16 || out_elem == MI_TILES_PARTS) && (row | 255) < gridDim.x)
+    row = (row & ~int64_t(255)) + (row & 7) * 32 + ((row >> 3) & 31);
+  const int64_t base = row * cols;
   auto quad = [&](const float *p, int64_t c, float pad) {
     f32x4u v;
     if (c + 4 <= cols) {
@@ -971,10 +996,12 @@ __global__ void __launch_bounds__(NTH) norm_block_kernel(const float *x, const f
     float *out = static_cast<float *>(out_any);
     if (out_elem == MI_F32 && c + 4 <= cols) {
       *reinterpret_cast<f32x4u *>(out + base + c) = y;
+    } else if (!LN && out_elem != MI_F32 && cols % 4 == 0) {
+      if (c < cols) norm_put4(out_any, out_elem, row, gridDim.x, c, cols, make_float4(y[0], y[1], y[2], y[3]));
     } else {
       for (int e = 0; e < 4 && c + e < cols; ++e) {
         if (LN || out_elem == MI_F32) out[base + c + e] = y[e];
-        else norm_put(out_any, out_elem, blockIdx.x, gridDim.x, c + e, cols, y[e]);
+        else norm_put(out_any, out_elem, row, gridDim.x, c + e, cols, y[e]);
       }
     }
   }

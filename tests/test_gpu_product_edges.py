@@ -110,7 +110,7 @@ def test_f32_any_shape_bias_residual(engine):
 # whole and with edges, each DMA width, k-tile remainders, one k-tile, slices.
 F32_SHAPES = [(64, 64, 32), (64, 64, 8), (65, 67, 33), (1, 1, 1), (130, 66, 20), (128, 192, 96), (512, 512, 512),
               (2048, 768, 256), (2050, 772, 260), (2049, 771, 259), (2048, 2048, 64), (2052, 2044, 68),
-              (257, 129, 2047), (1500, 1500, 300), (2048, 2048, 512)]
+              (257, 129, 2047), (1500, 1500, 300)]
 
 
 def _f32_product(engine, a, ta, b, tb):
@@ -289,9 +289,56 @@ def test_f32_small_operands(engine, m, n, k, ta, tb, small):
 
 @pytest.mark.parametrize("m,n,k", [(2048, 2048, 512), (1500, 1500, 300), (2048, 768, 256), (2049, 771, 259)])
 def test_f32_non_finite_operands_on_every_parts_tile(engine, m, n, k):
-    """As test_f32_non_finite_operands, on 128 x 128 tiles whole and with edges,
-    64 x 128 ones, and by 4-byte DMA."""
-    test_f32_non_finite_operands(engine, m, n, k)
+    """An infinity, a NaN and a value next to the largest on 128 x 128 tiles
+    whole and with edges, 64 x 128 ones, and by 4-byte DMA; the finite results
+    within an F32 sum's bound."""
+    rng = np.random.default_rng(n)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[3, 5], a[7, 1], a[9, 2], a[m - 1, k - 1] = np.inf, np.nan, np.float32(3.4028e38), -np.inf
+    b[5, 4] = b[2, 11] = 0.0
+    b[2] *= 0.125
+    got = _f32_product(engine, a, False, b, False)
+    with np.errstate(all="ignore"):
+        want, mag = a.astype(np.float64) @ b, np.abs(a).astype(np.float64) @ np.abs(b)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf, fin = np.isinf(want), np.isfinite(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32))
+    assert np.all(np.abs(got[fin] - want[fin]) <= (k + 4) * 2.0 ** -24 * mag[fin])
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_f32_product_on_whole_128_tiles(engine, ta, tb):
+    m, n, k = 2048, 2048, 512
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    got = _f32_product(engine, a.T.copy() if ta else a, ta, b.T.copy() if tb else b, tb)
+    av, bv = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(got - av @ bv) <= (k + 4) * 2.0 ** -24 * (np.abs(av) @ np.abs(bv)))
+
+
+@pytest.mark.parametrize("rows,cols", [(32, 2064), (288, 4096), (512, 3008), (544, 8192), (3, 2049), (5, 4098), (7, 2052)])
+def test_wide_rms_norm_forms_are_its_f32_result(engine, rows, cols):
+    """BF16, parts and tiled results of a block-a-row RMSNorm: the F32 result
+    rounded, its heads and remainders, and the same in tiles, bit for bit."""
+    rng = np.random.default_rng(cols)
+    x, g = (engine.upload(rng.standard_normal(d).astype(np.float32)) for d in ((rows, cols), (1, cols)))
+    y = engine.rms_norm(x, g)
+    yv = engine.download(y)
+    hi = bf16_bits(yv)
+    lo = bf16_bits(yv - bf16_to_f32(hi))
+    ids = [x, g, y]
+
+    def form(f):
+        ids.append(engine.rms_norm(x, g, 1e-5, f))
+        return engine.download(ids[-1])
+    assert np.array_equal(form(miburn.BF16), hi)
+    assert np.array_equal(form(miburn.BF16_PARTS), np.concatenate([hi, lo], 1))
+    if rows % 32 == 0 and cols % 16 == 0:
+        for f in (miburn.TILES_BF16, miburn.TILES_PARTS):
+            ids.append(engine.tile(y, f))
+            assert np.array_equal(form(f).reshape(-1), engine.download(ids[-2]).reshape(-1))
+    for t in ids:
+        engine.free(t)
 
 
 # ----------------------------------------------- more rows than one launch
