@@ -2102,18 +2102,17 @@ struct AnyTile {
 };
 static const AnyTile ANY_TILES[4] = {{128, 128, 0.33}, {192, 128, 0.41}, {256, 128, 0.50}, {256, 256, 0.83}};
 
+// Estimated time (us) of the product's tiles at ANY_TILES[t].
+static double any_us(const Plan &q, int t) {
+  const AnyTile &a = ANY_TILES[t];
+  const int64_t tiles = ((q.M + a.bm - 1) / a.bm) * ((q.N + a.bn - 1) / a.bn) * q.batch;
+  return static_cast<double>((tiles + 255) / 256) * (q.K / 32 * a.c + 1.5);
+}
+
 static int any_tile(const Plan &q) {
   int best = 0;
-  double least = 0;
-  for (int t = 0; t < 4; ++t) {
-    const AnyTile &a = ANY_TILES[t];
-    const int64_t tiles = ((q.M + a.bm - 1) / a.bm) * ((q.N + a.bn - 1) / a.bn) * q.batch;
-    const double us = static_cast<double>((tiles + 255) / 256) * (q.K / 32 * a.c + 1.5);
-    if (t == 0 || us < least) {
-      best = t;
-      least = us;
-    }
-  }
+  for (int t = 1; t < 4; ++t)
+    if (any_us(q, t) < any_us(q, best)) best = t;
   return best;
 }
 
@@ -2152,22 +2151,38 @@ static bool b_in_place(const Plan &p) {
   return p.eb == MI_BF16 && (p.tb || p.N % 8 == 0) && lies_for_dma(p, p.b, p.ldb, p.sb);
 }
 
-// A BF16 product off the whole tiles: the time of the guarded 64 x 64 tiles
-// (125 TF/s over a full chip of 16-byte chunks, 30 where the pitch puts rows
-// off them and every element is loaded by itself) against the direct kernel's
-// (450 TF/s) and its packs' (3 us and the bytes at 4 TB/s each); fewer tiles
-// than fill the chip cost either about the square root of what they leave
-// idle (split-K, the clock).
+// A BF16 product off the whole tiles: the time of the 64 x 64 register tiles
+// against the direct kernel's with its packs.  The register kernel takes 3 us
+// and, a k-tile of 64, the larger of a chain's latency and its blocks' loads:
+// least for operands with their k contiguous in 16-byte chunks, more for one
+// that has its rows contiguous, and for one off chunks, loaded element by
+// element; less where the tiles are exact; the direct kernel 3.5 us, its tiles' estimate, and for each operand it packs 2.5
+// us and the bytes at 4 TB/s; either its result at 8 TB/s.  us, register / direct:
+// with B^T 1000^3 17.3 / 21.8, 1728 x 1632 x 696 16.5 / 21.9, 3648 x 1088 x 448
+// 10.9 / 12.9, 2408 x 800 x 128 5.9 / 7.3, 1984 x 1728 x 1088 19.9 / 16.2, 1448 x
+// 2580 x 1704 42.0 / 33.8; as it lies 3016 x 848 x 568 28.9 / 18.8; off chunks
+// 645 x 2520 x 180 with B^T 11.9 / 13.0, 502 x 1330 x 806 37.6 / 19.4, 2105 x 448
+// x 64 with A^T 7.9 / 10.6.
 static bool bf16_any_pays(const Plan &p, int64_t t128) {
   const bool chunks = p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sa % 8 == 0 && p.sb % 8 == 0 &&
                       !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15);
   if (t128 < (chunks ? 32 : 8)) return false;
-  const double flop = 2.0 * static_cast<double>(p.M) * p.N * p.K * p.batch;
-  const double t64 = static_cast<double>(((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch);
-  const double guarded = flop / ((chunks ? 125e6 : 30e6) * std::min(1.0, std::sqrt(t64 / 1024)));
-  double direct = 1.5 + flop / (450e6 * std::min(1.0, std::sqrt(static_cast<double>(t128) / 256)));
-  if (!a_in_place(p)) direct += 3 + static_cast<double>(p.M * p.K * (p.sa ? p.batch : 1)) * 4 / 4e6;
-  if (!b_in_place(p)) direct += 3 + static_cast<double>(p.N * p.K * (p.sb ? p.batch : 1)) * 4 / 4e6;
+  const bool exact = tiles_exactly(p, 64, 64, 64, 8);
+  const double blocks = static_cast<double>(((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch) / 256;  // a CU
+  double lat = exact ? 0.95 : 1.15, load = exact ? 0.29 : 0.36;
+  auto operand = [&](bool kcontig, bool chunk) {
+    if (!exact) lat += kcontig ? (chunk ? 0.0 : 0.75) : (chunk ? 0.9 : 2.2);
+    load += kcontig ? (chunk ? 0.0 : 0.65) : (chunk ? 0.32 : 1.0);
+  };
+  operand(!p.ta, p.lda % 8 == 0 && p.sa % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.a) & 15));
+  operand(p.tb, p.ldb % 8 == 0 && p.sb % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.b) & 15));
+  const double out = static_cast<double>(p.M * p.N * p.batch) * 4;
+  const double guarded = 3 + static_cast<double>((p.K + 63) / 64) * std::max(lat, load * blocks) + out / 8e6;
+  Plan q = p;
+  q.K = (p.K + 31) / 32 * 32;
+  double direct = 3.5 + any_us(q, any_tile(q)) + out / 8e6;
+  if (!a_in_place(p)) direct += 2.5 + static_cast<double>(p.M * p.K * (p.sa ? p.batch : 1)) * 4 / 4e6;
+  if (!b_in_place(p)) direct += 2.5 + static_cast<double>(p.N * p.K * (p.sb ? p.batch : 1)) * 4 / 4e6;
   return direct < guarded;
 }
 
@@ -2182,7 +2197,7 @@ static bool bf16_any_pays(const Plan &p, int64_t t128) {
 //    93 -> 31; 2000 x 576 x 1536 37.7 -> 40.0, below the line at 2^31.
 //  * BF16 off the whole tiles, by bf16_any_pays: 2001^3 450 -> 38.8, 4095 x
 //    4097 x 4001 1719 -> 200 (transposed A 5180 -> 202), 1000^3 42.6 -> 21.3,
-//    700^3 29.2 -> 17.1, 512 x 512 x 500 19.8 -> 12.7; 2134 x 1840 x 136 (8.7
+//    700^3 29.2 -> 17.1, 512 x 512 x 500 19.8 -> 12.2; 2134 x 1840 x 136 (8.7
 //    against 13.0) and 100 x 3000 x 1000 (16.4 against 20.9) stay.
 static bool direct_any_pays(const Plan &p) {
   if (p.per_group || p.kc || p.swiglu || p.qkv.mode || p.M < 16 || p.N < 16) return false;
