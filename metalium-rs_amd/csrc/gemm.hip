@@ -1629,26 +1629,29 @@ static hipError_t run_f32(const Plan &p, hipStream_t st) {
   return launch_orient<T, SA, SB, TO, 64, 64, 2, 2, true>(p, st);
 }
 
+// The fast mode splits F32 operands where the product is large enough to be
+// bound by the matrix cores (at least 2^33 multiply-adds over at least 128
+// tiles of 128 x 128): below that the kernels are bound by load latency and
+// the split's conversions only add work, so the F32 kernel runs (more
+// accurate, and faster there).
+// F32 activations against BF16 weights over at least 256 rows are the
+// exception at any size: split, only the activations take two BF16 parts,
+// and the k loop runs on the BF16 matrix cores instead of the F32 ones (a
+// 512-token prefill of the SmolLM2-shaped decoder 8.7 -> 7.5 ms; its
+// products at 2048 - 8192 rows, us: gate|up at 2048 rows 86.6 -> 42.0, down
+// at 4096 98.7 -> 39.8, down at 8192 167.7 -> 81.7, o at 8192 66.9 -> 38.0).
+static bool split_pays(const Plan &p) {
+  if (!p.fast || (p.ea != MI_F32 && p.eb != MI_F32)) return false;
+  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return true;
+  return p.M * p.N * p.K * p.batch >= (int64_t(1) << 33) &&
+         ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch >= 128;
+}
+
 static hipError_t run_plan(const Plan &p, hipStream_t st) {
   const bool bf = p.eo == MI_BF16;
   if (p.ea == MI_BF16 && p.eb == MI_BF16)
     return bf ? run_bf16<uint16_t>(p, st) : run_bf16<float>(p, st);
-  // The fast mode splits F32 operands where the product is large enough to be
-  // bound by the matrix cores (at least 2^33 multiply-adds over at least 128
-  // tiles of 128 x 128): below that the kernels are bound by load latency and
-  // the split's conversions only add work, so the F32 kernel runs (more
-  // accurate, and faster there).
-  // F32 activations against BF16 weights over at least 256 rows are the
-  // exception at any size: split, only the activations take two BF16 parts,
-  // and the k loop runs on the BF16 matrix cores instead of the F32 ones (a
-  // 512-token prefill of the SmolLM2-shaped decoder 8.7 -> 7.5 ms; its
-  // products at 2048 - 8192 rows, us: gate|up at 2048 rows 86.6 -> 42.0, down
-  // at 4096 98.7 -> 39.8, down at 8192 167.7 -> 81.7, o at 8192 66.9 -> 38.0).
-  const int64_t macs = p.M * p.N * p.K * p.batch;
-  const bool split_pays =
-      (macs >= (int64_t(1) << 33) && ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch >= 128) ||
-      (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256);
-  if (p.fast && split_pays) {
+  if (split_pays(p)) {
     if (p.ea == MI_F32 && p.eb == MI_F32)
       return bf ? run_split<float, float, uint16_t>(p, st) : run_split<float, float, float>(p, st);
     if (p.ea == MI_F32)
@@ -1725,7 +1728,8 @@ static bool split_slices(const Plan &p) {
 // 16 us in 16 slices; the MLP's [64, 784] x [784, 128] gains from 6).
 static int splitk_slices(const Plan &p) {
   if (p.batch != 1) return 1;
-  if (f32_pipe_fits(p)) return f32_pipe_slices(p);
+  // (Whole where the split kernel has two blocks a CU or more.)
+  if (f32_pipe_fits(p)) return split_pays(p) && ((p.M + 63) / 64) * ((p.N + 63) / 64) >= 512 ? 1 : f32_pipe_slices(p);
   // BF16 operands tiled exactly by 128 run the pipelined kernel whole once
   // its tiles (16 or more) cover the k loop, tiles x 128 >= k: 1024^3 in
   // 11 us against 26 us split four ways on the register kernel, 768 x 768
@@ -2199,6 +2203,11 @@ static bool bf16_any_pays(const Plan &p, int64_t t128) {
 //    4097 x 4001 1719 -> 200 (transposed A 5180 -> 202), 1000^3 42.6 -> 21.3,
 //    700^3 29.2 -> 17.1, 512 x 512 x 500 19.8 -> 12.2; 2134 x 1840 x 136 (8.7
 //    against 13.0) and 100 x 3000 x 1000 (16.4 against 20.9) stay.
+//  * F32 against B^T in whole 64 x 64 tiles stays on the split kernel up to two
+//    of them a CU (2048 x 1024 x 8192 204 against 241, 1024 x 2048 x 4160 106
+//    against 128; past that 1536 x 1536 x 8192 371 against 242), three against
+//    BF16 (2048 x 1024 x 1024 21.0 against 33.7, 1536 x 2048 x 1024 27.0 against
+//    33.2; past that 1920 x 1920 x 1024 38.0 against 31.9).
 static bool direct_any_pays(const Plan &p) {
   if (p.per_group || p.kc || p.swiglu || p.qkv.mode || p.M < 16 || p.N < 16) return false;
   const bool f32 = p.ea == MI_F32 || p.eb == MI_F32;
@@ -2211,7 +2220,9 @@ static bool direct_any_pays(const Plan &p) {
   // 777 x 3001 1.3e-7 against 3.3e-7), whatever it takes (34.1 us against 28.8,
   // 123 against 40.8; 300 x 300 x 3001 18.2 against 37.8).
   if (!f32) return splitk_slices(p) <= 1 && bf16_any_pays(p, t128);
-  if (p.batch == 1 && ((p.M + 63) / 64) * ((p.N + 63) / 64) < 512) return false;
+  const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+  if (p.batch == 1 && t64 < 512) return false;
+  if (!p.ta && p.tb && t64 <= (p.eb == MI_BF16 ? 768 : 512) && tiles_exactly(p, 64, 64, 64, 8)) return false;
   if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return macs >= (int64_t(1) << 31) && t128 >= 128;
   return macs >= (int64_t(1) << 33) && t128 >= 128;
 }
