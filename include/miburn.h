@@ -302,18 +302,21 @@ int mi_linear_qkv_rope_cache(mi_ctx *ctx, mi_id x, int x_parts, mi_id w_qkv,
  * operand; BF16 x BF16 products are the same in both.
  *  FAST (the default, as the reference's): where a product is large enough to
  *   be bound by the matrix cores (>= 2^33 multiply-adds over >= 128 tiles of
- *   128 x 128), and for F32 activations (>= 256 rows) against BF16 weights at
- *   any size, each F32 operand element is split as bf16 hi + bf16 lo and
+ *   128 x 128), and for F32 activations (>= MI_SPLIT_MIN_ROWS rows) against BF16
+ *   weights at any size, each F32 operand element is split as bf16 hi + bf16 lo and
  *   a b = hi hi + hi lo + lo hi runs on the BF16 matrix cores with F32
  *   accumulation (hi b + lo b for a BF16 b); error per product <= 3 * 2^-18
  *   |a||b| (the reference's fast mode rounds operands to TF32, 2^-11).  Other
  *   products run as in ACCURATE.  A non-finite operand element gives NaN in
  *   its row or column where F32 arithmetic could give an infinity.
  *  ACCURATE: F32 products at F32 precision, F32 accumulation: on the F32 matrix
- *   cores, or on the BF16 ones with each element in three parts (24 bits).
+ *   cores, or on the BF16 ones with each element in three parts (24 bits; tiles
+ *   with a value that three cannot hold are formed on the F32 ones).
  * The reference's EXACT mode (k-ordered sequential F32 sums) is not offered:
  * MI_E_UNSUPPORTED. ---- */
 enum mi_matmul_mode { MI_MATMUL_FAST = 0, MI_MATMUL_ACCURATE = 1 };
+/* The rows from which FAST splits F32 activations against BF16 weights. */
+enum { MI_SPLIT_MIN_ROWS = 256 };
 int mi_set_matmul_mode(mi_ctx *ctx, int mode);
 int mi_get_matmul_mode(mi_ctx *ctx, int *mode);
 

@@ -1642,7 +1642,7 @@ static hipError_t run_f32(const Plan &p, hipStream_t st) {
 // at 4096 98.7 -> 39.8, down at 8192 167.7 -> 81.7, o at 8192 66.9 -> 38.0).
 static bool split_pays(const Plan &p) {
   if (!p.fast || (p.ea != MI_F32 && p.eb != MI_F32)) return false;
-  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return true;
+  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= MI_SPLIT_MIN_ROWS) return true;
   return p.M * p.N * p.K * p.batch >= (int64_t(1) << 33) &&
          ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch >= 128;
 }
@@ -1717,7 +1717,7 @@ static void launch_gemv(const Plan &p, hipStream_t st) {
 // Whether a sliced product runs on the split kernel: F32 activations (256 or
 // more rows) against a BF16 weight in the fast mode.
 static bool split_slices(const Plan &p) {
-  return p.fast && p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256;
+  return p.fast && p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= MI_SPLIT_MIN_ROWS;
 }
 
 // Split-K for few output tiles over a long k: enough (tile, slice) pairs to
@@ -2223,7 +2223,7 @@ static bool direct_any_pays(const Plan &p) {
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
   if (p.batch == 1 && t64 < 512) return false;
   if (!p.ta && p.tb && t64 <= (p.eb == MI_BF16 ? 768 : 512) && tiles_exactly(p, 64, 64, 64, 8)) return false;
-  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= 256) return macs >= (int64_t(1) << 31) && t128 >= 128;
+  if (p.ea == MI_F32 && p.eb == MI_BF16 && p.M >= MI_SPLIT_MIN_ROWS) return macs >= (int64_t(1) << 31) && t128 >= 128;
   return macs >= (int64_t(1) << 33) && t128 >= 128;
 }
 

@@ -140,8 +140,6 @@ constexpr int64_t kSpanStep = 64;
 constexpr int64_t kTilesMaxRows = 2048;
 // New positions from which a prompt is padded to run on them.
 constexpr int64_t kPadMinT = 17;
-// Rows from which the fast mode splits F32 activations against BF16 weights.
-constexpr int64_t kSplitMinRows = 256;
 
 // The caches and rotary tables hold max_ctx positions rounded up to this, so
 // that a prompt reaching max_ctx can be run a few padding positions longer.
@@ -233,7 +231,7 @@ int64_t padded_positions(const mi_llama *m, int64_t batch, int64_t t, int64_t po
   if (t < kPadMinT || m->layers.empty() || !m->layers[0].t_wqkv.defined()) return t;
   int mode = MI_MATMUL_FAST;
   (void)mi_get_matmul_mode(m->ctx, &mode);
-  if (c.numerics != MI_NUMERICS_PERFORMANCE && (mode != MI_MATMUL_FAST || batch * t < kSplitMinRows)) return t;
+  if (c.numerics != MI_NUMERICS_PERFORMANCE && (mode != MI_MATMUL_FAST || batch * t < MI_SPLIT_MIN_ROWS)) return t;
   int64_t tp = t;
   while (batch * tp % 32) ++tp;
   return batch * tp <= kTilesMaxRows && pos0 + tp <= cache_cap(c) ? tp : t;
