@@ -2156,37 +2156,39 @@ static bool b_in_place(const Plan &p) {
 }
 
 // A BF16 product off the whole tiles: the time of the 64 x 64 register tiles
-// against the direct kernel's with its packs.  The register kernel takes 3 us
+// against the direct kernel's with its packs.  The register kernel takes 2.6 us
 // and, a k-tile of 64, the larger of a chain's latency and its blocks' loads:
 // least for operands with their k contiguous in 16-byte chunks, more for one
 // that has its rows contiguous, and for one off chunks, loaded element by
-// element; less where the tiles are exact; the direct kernel 3.5 us, its tiles' estimate, and for each operand it packs 2.5
-// us and the bytes at 4 TB/s; either its result at 8 TB/s.  us, register / direct:
+// element; less where the tiles are exact; the direct kernel 2.6 us, its tiles'
+// estimate, and for each operand it packs 2.5 us and the bytes at 4.9 TB/s;
+// either its result at 8 TB/s.  The constants are fitted to both sides of 420
+// drawn shapes: 0.3% over the faster side in the mean, over 5% at 13 of them and
+// a quarter at worst (2009 x 744 x 304 17.2 / 13.8).  us, register / direct:
 // with B^T 1000^3 17.3 / 21.8, 1728 x 1632 x 696 16.5 / 21.9, 3648 x 1088 x 448
 // 10.9 / 12.9, 2408 x 800 x 128 5.9 / 7.3, 1984 x 1728 x 1088 19.9 / 16.2, 1448 x
 // 2580 x 1704 42.0 / 33.8; as it lies 3016 x 848 x 568 28.9 / 18.8; off chunks
-// 645 x 2520 x 180 with B^T 11.9 / 13.0, 502 x 1330 x 806 37.6 / 19.4, 2105 x 448
-// x 64 with A^T 7.9 / 10.6.
+// with B^T 502 x 1330 x 806 37.6 / 19.4.
 static bool bf16_any_pays(const Plan &p, int64_t t128) {
   const bool chunks = p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sa % 8 == 0 && p.sb % 8 == 0 &&
                       !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.b) & 15);
   if (t128 < (chunks ? 32 : 8)) return false;
   const bool exact = tiles_exactly(p, 64, 64, 64, 8);
   const double blocks = static_cast<double>(((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch) / 256;  // a CU
-  double lat = exact ? 0.95 : 1.15, load = exact ? 0.29 : 0.36;
+  double lat = exact ? 0.8 : 1.15, load = exact ? 0.26 : 0.36;
   auto operand = [&](bool kcontig, bool chunk) {
-    if (!exact) lat += kcontig ? (chunk ? 0.0 : 0.75) : (chunk ? 0.9 : 2.2);
-    load += kcontig ? (chunk ? 0.0 : 0.65) : (chunk ? 0.32 : 1.0);
+    if (!exact) lat += kcontig ? (chunk ? 0.0 : 0.75) : (chunk ? 0.93 : 2.85);
+    load += kcontig ? (chunk ? 0.0 : 0.72) : (chunk ? 0.57 : 1.0);
   };
   operand(!p.ta, p.lda % 8 == 0 && p.sa % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.a) & 15));
   operand(p.tb, p.ldb % 8 == 0 && p.sb % 8 == 0 && !(reinterpret_cast<uintptr_t>(p.b) & 15));
   const double out = static_cast<double>(p.M * p.N * p.batch) * 4;
-  const double guarded = 3 + static_cast<double>((p.K + 63) / 64) * std::max(lat, load * blocks) + out / 8e6;
+  const double guarded = 2.6 + static_cast<double>((p.K + 63) / 64) * std::max(lat, load * blocks) + out / 8e6;
   Plan q = p;
   q.K = (p.K + 31) / 32 * 32;
-  double direct = 3.5 + any_us(q, any_tile(q)) + out / 8e6;
-  if (!a_in_place(p)) direct += 2.5 + static_cast<double>(p.M * p.K * (p.sa ? p.batch : 1)) * 4 / 4e6;
-  if (!b_in_place(p)) direct += 2.5 + static_cast<double>(p.N * p.K * (p.sb ? p.batch : 1)) * 4 / 4e6;
+  double direct = 2.6 + any_us(q, any_tile(q)) + out / 8e6;
+  if (!a_in_place(p)) direct += 2.5 + static_cast<double>(p.M * p.K * (p.sa ? p.batch : 1)) * 4 / 4.9e6;
+  if (!b_in_place(p)) direct += 2.5 + static_cast<double>(p.N * p.K * (p.sb ? p.batch : 1)) * 4 / 4.9e6;
   return direct < guarded;
 }
 
