@@ -19,11 +19,11 @@
 //    other's products.
 //
 // us, against the register-staged 64 x 64 / 128 x 128 kernel it replaces:
-// 4096^3 (accurate mode) 1075 -> 809 (170 TF/s; 762 at best), 2048 x 8192 x 256
-// 82 -> 63, [256, 8192] over k 2000 transposed 138 -> 71, 16 x 512^3 44.0 ->
-// 33.9, 1500^3 128 -> 65, 512^3 15.0 -> 9.6, 64 x 128 x 784 12.4 -> 9.5.  The
-// error against float64 falls at each (4096^3 1.1e-6 -> 1.0e-6, 1500^3 6.9e-7
-// -> 3.4e-7).
+// 4096^3 (accurate mode) 1059 -> 747 (184 TF/s; 737 at best), 2048 x 8192 x 256
+// 79 -> 59, [256, 8192] over k 2000 transposed 138 -> 69, 16 x 512^3 44.0 ->
+// 32.2, 1500^3 128 -> 63, 512^3 15.4 -> 10.4, 64 x 128 x 784 12.7 -> 9.8.  The
+// error against float64 falls at each (4096 x 4096 x 512 4.1e-7 -> 3.4e-7, 2048
+// x 768 x 256 2.9e-7 -> 1.7e-7).
 //
 // LDS tiles.  An operand whose k is contiguous lies as 128-byte rows of 32 k
 // in 16-byte chunks, chunk c of row r at c ^ (r / 2 & 7); a lane's fragment is one
