@@ -421,8 +421,8 @@ def test_ragged_prompt_runs_padded(engine, batch, t, longer, numerics):
     full.close()
 
 
-@pytest.mark.parametrize("batch,t,numerics", [(1, 300, "reference"), (3, 100, "reference"), (1, 17, "performance"),
-                                              (2, 33, "performance")])
+@pytest.mark.parametrize("batch,t,numerics", [(1, 300, "reference"), (3, 100, "reference"), (1, 100, "performance"),
+                                              (2, 75, "performance")])
 def test_ragged_prompt_without_eps(engine, batch, t, numerics):
     """eps 0: the padding rows of a ragged prompt are finite, so its last
     positions, whose key block they share, are what the CPU model gives."""

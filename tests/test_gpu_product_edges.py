@@ -268,19 +268,21 @@ def test_f32_short_k_is_f32_arithmetic(engine, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(2048, 768, 256), (2048, 2048, 512), (1500, 1500, 300), (2049, 771, 259),
                                    (256, 512, 2065)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
-@pytest.mark.parametrize("small", ["a", "b", "a few"])
+@pytest.mark.parametrize("small", ["a", "b", "one column", "subnormal"])
 def test_f32_small_operands(engine, m, n, k, ta, tb, small):
     """Values whose last bits lie below BF16's least subnormal (2^-133), down to
     F32's own subnormals, against ones that bring their products to ordinary
     size: an F32 sum's bound, as for any other values."""
     rng = np.random.default_rng(m + k)
     a, b = rng.standard_normal((m, k)), rng.standard_normal((k, n))
-    if small == "a few":  # one column of A below, its row of B far above the rest
-        a[:, 5] = np.ldexp(a[:, 5], -118)
-        b[5] = np.ldexp(b[5], 118)
+    if small == "one column":  # of A, and its row of B far above the rest
+        a[:, 5] = np.ldexp(a[:, 5], -124)
+        b[5] = np.ldexp(b[5], 124)
+        b[:5], b[6:] = b[:5] * 2.0 ** -30, b[6:] * 2.0 ** -30
+    elif small == "b":
+        a, b = np.ldexp(a, 100), np.ldexp(b, -124)
     else:
-        e = rng.integers(-130, -108, (1, k))
-        a, b = (np.ldexp(a, e), np.ldexp(b, 110)) if small == "a" else (np.ldexp(a, 110), np.ldexp(b, e.T))
+        a, b = np.ldexp(a, -124 if small == "a" else -132), np.ldexp(b, 100)
     a, b = a.astype(np.float32), b.astype(np.float32)
     got = _f32_product(engine, a.T.copy() if ta else a, ta, b.T.copy() if tb else b, tb)
     av, bv = a.astype(np.float64), b.astype(np.float64)
