@@ -264,9 +264,10 @@ def test_f32_short_k_is_f32_arithmetic(engine, m, n, k):
     assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b)) * (1 + 2.0 ** -20))
 
 
-# 64 x 128 and 128 x 128 tiles, whole, with edges and by 4-byte DMA, and slices.
+# 64 x 128 and 128 x 128 tiles, whole, with edges and by 4-byte DMA; 64 x 128 in
+# slices, the last of them one k-tile of 4.
 @pytest.mark.parametrize("m,n,k", [(2048, 768, 256), (2048, 2048, 512), (1500, 1500, 300), (2049, 771, 259),
-                                   (256, 512, 2065)])
+                                   (256, 768, 2308)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
 @pytest.mark.parametrize("small", ["a", "b", "one column", "subnormal"])
 def test_f32_small_operands(engine, m, n, k, ta, tb, small):
@@ -308,14 +309,16 @@ def test_f32_non_finite_operands_on_every_parts_tile(engine, m, n, k):
     assert np.all(np.abs(got[fin] - want[fin]) <= (k + 4) * 2.0 ** -24 * mag[fin])
 
 
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 512), (256, 768, 2308)])  # 128 x 128 whole; a slice of one k-tile
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
-def test_f32_product_on_whole_128_tiles(engine, ta, tb):
-    m, n, k = 2048, 2048, 512
+def test_f32_product_on_parts_tiles(engine, m, n, k, ta, tb):
     rng = np.random.default_rng(k)
     a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
     got = _f32_product(engine, a.T.copy() if ta else a, ta, b.T.copy() if tb else b, tb)
     av, bv = a.astype(np.float64), b.astype(np.float64)
     assert np.all(np.abs(got - av @ bv) <= (k + 4) * 2.0 ** -24 * (np.abs(av) @ np.abs(bv)))
+    again = _f32_product(engine, a.T.copy() if ta else a, ta, b.T.copy() if tb else b, tb)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
 
 
 @pytest.mark.parametrize("rows,cols", [(32, 2064), (288, 4096), (512, 3008), (544, 8192), (3, 2049), (5, 4098), (7, 2052)])
