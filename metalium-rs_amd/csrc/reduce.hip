@@ -47,9 +47,9 @@ __device__ __forceinline__ float fold_op(int op, float a, float b) {
 
 // One wavefront per row; four rows per 256-thread block.  Four chains a lane,
 // each over every fourth load: as many loads in flight, and sums of a quarter
-// the length.  The op is fixed at compile time: tested in the loop, the chains
-// ran twice as long as one (512 x 8192 2.0, now 0.91 of one chain's 4.9 us;
-// 16384 x 513 9.3 -> 5.6, 8191 x 4095 27.2 -> 20.5).
+// the length.  The op is fixed at compile time (tested in the loop, four chains
+// take twice the time of one).  us, one chain / four: 512 x 8192 4.9 / 4.4,
+// 16384 x 513 9.3 / 5.6, 8191 x 4095 27.2 / 20.5.
 template <bool NT, int op>
 __global__ void __launch_bounds__(256) reduce_cols_kernel(const void *x, int elem, float *out, int64_t rows,
                                                           int64_t cols) {
